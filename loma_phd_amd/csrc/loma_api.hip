@@ -419,40 +419,55 @@ int loma_init(loma_run** out, int mgalx, int my, int mgalz, const double* y, dou
   // the kernels address with constant offsets
   const size_t tot = ytab_offset(YT_COUNT, M);
   std::vector<double> h(tot, 0.0);
-  auto lm = [&](int row, int w, int idx) -> size_t {
-    const int l = row / M, t = row - l * M;
-    return (size_t)(t * w + idx) * 64 + l;
+  std::vector<float> h32(tot, 0.0f);
+  // entry e of lane l in table `id` (its stream at element `o` holds n
+  // entries a lane), in the FP64 and the FP32 vector layout
+  auto set = [&](size_t o, int n, int e, int l, double v) {
+    h[o + stream_index(n, e, l, 2)] = v;
+    h32[o + stream_index(n, e, l, 4)] = (float)v;
   };
-  // row-indexed table -> lane-major
-  auto put = [&](int id, const std::vector<double>& src) {
-    const int w = ytab_width(id);
-    const size_t o = ytab_offset(id, M);
+  auto put_at = [&](int id, int row, int idx, double v) {
+    const int w = ytab_width(id), l = row / M, t = row - l * M;
+    set(ytab_offset(id, M), w * M, t * w + idx, l, v);
+  };
+  // row-indexed source -> table entries i0 .. i0+w-1 of each row
+  auto put = [&](int id, const std::vector<double>& src, int w, int i0) {
     for (int j = 0; j < my; ++j)
-      for (int d = 0; d < w; ++d) h[o + lm(j, w, d)] = src[(size_t)j * w + d];
+      for (int d = 0; d < w; ++d) put_at(id, j, i0 + d, src[(size_t)j * w + d]);
   };
   // lower multipliers: lo[k][i-1] (row k into row k+i) -> destination row k+i
   auto put_lo = [&](int id, const std::vector<double>& src) {
     const int w = ytab_width(id);
-    const size_t o = ytab_offset(id, M);
     for (int j = 0; j < my; ++j)
       for (int i = 1; i <= w; ++i)
-        if (j - i >= 0) h[o + lm(j, w, i - 1)] = src[(size_t)(j - i) * w + i - 1];
+        if (j - i >= 0) put_at(id, j, i - 1, src[(size_t)(j - i) * w + i - 1]);
   };
-  put(YT_B1, f.b1); put(YT_A1, f.a1); put(YT_INV1, f.inv1); put(YT_UP1, f.up1);
-  put_lo(YT_LO1, f.lo1); put(YT_FMAP, f.fmap); put(YT_B2, f.b2); put(YT_A2, f.a2);
-  put(YT_INV2, f.inv2); put(YT_UP2, f.up2); put_lo(YT_LO2, f.lo2); put(YT_INVI, f.invi);
-  put(YT_UPI, f.upi); put_lo(YT_LOI, f.loi); put(YT_WBD, wbd);
-  auto H = [&](int id) { return h.data() + ytab_offset(id, M); };
+  put(YT_B1, f.b1, 7, 0); put(YT_A1, f.a1, 7, 0); put(YT_U1, f.inv1, 1, 0);
+  put(YT_U1, f.up1, 3, 1); put_lo(YT_LO1, f.lo1); put(YT_FMAP, f.fmap, 1, 0);
+  put(YT_B2, f.b2, 5, 0); put(YT_A2, f.a2, 5, 0); put(YT_U2, f.inv2, 1, 0);
+  put(YT_U2, f.up2, 2, 1); put_lo(YT_LO2, f.lo2); put(YT_UI, f.invi, 1, 0);
+  put(YT_UI, f.upi, 3, 1); put_lo(YT_LOI, f.loi); put(YT_WBD, wbd, 2, 0);
+  // scan compositions, [level][P*P][lane] -> one stream a level
+  std::vector<double> hs((size_t)6 * 9 * 64);
+  auto scan = [&](int id, bool upper, const double* lo, const double* up, const double* inv) {
+    const int P = ytab_width(id);
+    const int lev = scan_table(my, M, P, upper, lo, up, inv, hs.data());
+    for (int k = 0; k < 6; ++k)
+      for (int e = 0; e < P * P; ++e)
+        for (int l = 0; l < 64; ++l)
+          set(ytab_offset(id, M) + (size_t)k * P * P * 64, P * P, e, l,
+              hs[((size_t)k * P * P + e) * 64 + l]);
+    return lev;
+  };
   int lev[6];
-  lev[0] = scan_table(my, M, 3, false, f.lo1.data(), nullptr, nullptr, H(YT_HL1));
-  lev[1] = scan_table(my, M, 3, true, nullptr, f.up1.data(), f.inv1.data(), H(YT_HU1));
-  lev[2] = scan_table(my, M, 2, false, f.lo2.data(), nullptr, nullptr, H(YT_HL2));
-  lev[3] = scan_table(my, M, 2, true, nullptr, f.up2.data(), f.inv2.data(), H(YT_HU2));
-  lev[4] = scan_table(my, M, 3, false, f.loi.data(), nullptr, nullptr, H(YT_HLI));
-  lev[5] = scan_table(my, M, 3, true, nullptr, f.upi.data(), f.invi.data(), H(YT_HUI));
-  // the FP64 tables, then their FP32 rounding in the same layout (the
-  // mixed form's FP32 y-operators read it)
-  std::vector<float> h32(h.begin(), h.end());
+  lev[0] = scan(YT_HL1, false, f.lo1.data(), nullptr, nullptr);
+  lev[1] = scan(YT_HU1, true, nullptr, f.up1.data(), f.inv1.data());
+  lev[2] = scan(YT_HL2, false, f.lo2.data(), nullptr, nullptr);
+  lev[3] = scan(YT_HU2, true, nullptr, f.up2.data(), f.inv2.data());
+  lev[4] = scan(YT_HLI, false, f.loi.data(), nullptr, nullptr);
+  lev[5] = scan(YT_HUI, true, nullptr, f.upi.data(), f.invi.data());
+  // the FP64 tables, then their FP32 rounding (the mixed form's FP32
+  // y-operators read it)
   if ((rc = dalloc(r, &r->tab, tot * (sizeof(double) + sizeof(float))))) {
     loma_free(r); return rc;
   }

@@ -9,11 +9,15 @@
 // reference's sequential banbks/banbks7 sweeps (cfdiff.f:954-1051) with all
 // 64 lanes busy.
 //
-// Per-row coefficient tables are stored lane-major: entry `idx` of row
-// (lane*M + t) sits at base[(t*ncol + idx)*64 + lane], so every table load of
-// a wavefront is one contiguous 512-byte segment.  Lower-triangle
-// multipliers are stored by destination row (lo(r, i-1) multiplies row r-i
-// into row r), so every lane reads only its own rows.
+// Coefficient tables are lane-major streams of 16-byte vectors: a lane's
+// entries in the order of its rows, two doubles (four floats) to a vector,
+// vector q of all lanes contiguous, the few entries that do not fill a vector
+// behind them (stream_index).  The y operators are bound by the rate of
+// vector-memory instructions (about 15 cycles per wavefront load and CU,
+// whatever its width or addresses), so a table is read 16 bytes a lane at a
+// time.  Lower-triangle multipliers are stored by destination row
+// (lo(r, i-1) multiplies row r-i into row r), so every lane reads only its
+// own rows.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -49,34 +53,21 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, in
                                            bytes < 0 ? 0 : bytes, RSRC_WORD3);
 }
 
-// lane-major table view: resource over the table, entries per row, first
-// entry used, this lane's byte offset and a scalar bias (see relaunder)
+// position of entry e of lane `lane` in a lane-major stream of n entries a
+// lane, vw entries to a 16-byte vector
+__host__ __device__ inline int stream_index(int n, int e, int lane, int vw) {
+  return e < n / vw * vw ? (e / vw * WAVE + lane) * vw + e % vw : e * WAVE + lane;
+}
+
+// view of a stream: resource over the allocation, this lane's byte offset in
+// a vector row and a scalar byte bias (the stream's offset; see relaunder)
 struct TabRef {
   __amdgpu_buffer_rsrc_t r;
-  int ncol;
-  int off;
   int lane_off;
   int sbias;
 };
-__device__ __forceinline__ TabRef tab(const double* base, int ncol, int off, int lane) {
-  return TabRef{make_rsrc(base, 0x7fffffff), ncol, off, lane * 8, 0};
-}
-__device__ __forceinline__ double tget(const TabRef& b, int t, int idx) {
-  const auto v = __builtin_amdgcn_raw_buffer_load_b64(
-      b.r, b.lane_off, b.sbias + (t * b.ncol + b.off + idx) * (WAVE * 8), 0);
-  return __builtin_bit_cast(double, v);
-}
-// entry of a table in the arithmetic type V: the FP64 table, or its FP32
-// copy (a view made by ytab_v<M, float>, whose lane offset counts 4 bytes)
-template <typename V>
-__device__ __forceinline__ V tget_v(const TabRef& b, int t, int idx) {
-  if constexpr (sizeof(V) == 8) {
-    return tget(b, t, idx);
-  } else {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b32(
-        b.r, b.lane_off, b.sbias + (t * b.ncol + b.off + idx) * (WAVE * 4), 0);
-    return __builtin_bit_cast(float, v);
-  }
+__device__ __forceinline__ TabRef tab(const double* base, int lane) {
+  return TabRef{make_rsrc(base, 0x7fffffff), lane * 16, 0};
 }
 // The same view, opaque to the optimiser: loads through it are issued again
 // instead of keeping coefficients loaded earlier live across a scan (table
@@ -84,7 +75,7 @@ __device__ __forceinline__ V tget_v(const TabRef& b, int t, int idx) {
 __device__ __forceinline__ TabRef relaunder(const TabRef& b) {
   int z = b.sbias;
   asm volatile("" : "+s"(z));
-  return TabRef{b.r, b.ncol, b.off, b.lane_off, z};
+  return TabRef{b.r, b.lane_off, z};
 }
 // The same, additionally ordered after `dep` is computed: a level of a scan
 // loads its table entries once the previous level's carry exists, all
@@ -94,36 +85,58 @@ template <typename V>
 __device__ __forceinline__ TabRef relaunder_after(const TabRef& b, V dep) {
   int z = b.sbias;
   asm volatile("" : "+s"(z) : "v"(dep));
-  return TabRef{b.r, b.ncol, b.off, b.lane_off, z};
+  return TabRef{b.r, b.lane_off, z};
 }
-// Entries [0, K) of row t of a table view, issued together, and the wait
-// for a row loaded ahead, taken once for the whole row: left to itself the
-// scheduler issues each coefficient load next to its product, one memory
-// round trip per coefficient.
-template <int K, typename V>
-__device__ __forceinline__ void row_ld(const TabRef& b, int t, V (&c)[K]) {
+
+// A lane's stream of ROWS rows of W entries in registers; only the vectors
+// asked for are loaded (every index folds at compile time).
+template <typename V, int W, int ROWS>
+struct RowStream {
+  static constexpr int VW = 16 / (int)sizeof(V), N = W * ROWS, NF = N / VW;
+  V e[N];
+  __device__ __forceinline__ V operator()(int t, int i) const { return e[t * W + i]; }
+  __device__ __forceinline__ void ld(const TabRef& b, int q) {
+    typedef V vec __attribute__((ext_vector_type(16 / sizeof(V))));
+    const vec v = __builtin_bit_cast(
+        vec, __builtin_amdgcn_raw_buffer_load_b128(b.r, b.lane_off, b.sbias + q * (WAVE * 16), 0));
 #pragma unroll
-  for (int i = 0; i < K; ++i) c[i] = tget_v<V>(b, t, i);
-}
-template <int K, typename V>
-__device__ __forceinline__ void row_take(const V (&n)[K], V (&c)[K]) {
-#pragma unroll
-  for (int i = 0; i < K; ++i) {
-    c[i] = n[i];
-    asm volatile("" : "+v"(c[i]));
+    for (int i = 0; i < VW; ++i) e[q * VW + i] = v[i];
   }
-}
-// index of entry `idx` of grid row `row` in a lane-major table
-template <int M>
-__host__ __device__ inline int lane_major_index(int row, int ncol, int idx) {
-  const int l = row / M, t = row - l * M;
-  return (t * ncol + idx) * WAVE + l;
-}
-// entry `idx` of grid row `row` (any lane's) of a lane-major table
-template <int M>
-__device__ __forceinline__ double trow(const double* base, int ncol, int idx, int row) {
-  return base[lane_major_index<M>(row, ncol, idx)];
-}
+  __device__ __forceinline__ void ld_tail(const TabRef& b, int k) {
+    const int lo = b.lane_off / VW, so = b.sbias + k * (WAVE * (int)sizeof(V));
+    if constexpr (sizeof(V) == 8)
+      e[k] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(b.r, lo, so, 0));
+    else
+      e[k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(b.r, lo, so, 0));
+  }
+  // the vectors whose first row (of those >= t0) is t: rows read upwards
+  __device__ __forceinline__ void up(const TabRef& b, int t, int t0 = 0) {
+#pragma unroll
+    for (int q = 0; q < NF; ++q) {
+      const int f = q * VW / W, l = (q * VW + VW - 1) / W;
+      if ((f > t0 ? f : t0) == t && l >= t0) ld(b, q);
+    }
+#pragma unroll
+    for (int k = NF * VW; k < N; ++k)
+      if (k / W == t) ld_tail(b, k);
+  }
+  // the vectors whose last row is t: rows read downwards
+  __device__ __forceinline__ void down(const TabRef& b, int t) {
+#pragma unroll
+    for (int k = N - 1; k >= NF * VW; --k)
+      if (k / W == t) ld_tail(b, k);
+#pragma unroll
+    for (int q = NF - 1; q >= 0; --q)
+      if ((q * VW + VW - 1) / W == t) ld(b, q);
+  }
+  // the wait for row t, taken once for the whole row: left to itself the
+  // scheduler issues each load next to its product, one memory round trip
+  // per load
+  __device__ __forceinline__ void take(int t) {
+#pragma unroll
+    for (int i = 0; i < W; ++i) asm volatile("" : "+v"(e[t * W + i]));
+  }
+};
 
 // ---- wavefront scans of affine maps s_out = A s_in + c -----------------
 template <int P, int NC>
@@ -224,15 +237,18 @@ template <int M, int P, int NC>
 __device__ __forceinline__ void lsolve(const TabRef lo, int lane, double (&x)[NC][M]) {
   static_assert(P <= M, "chunk shorter than bandwidth");
   // (1) in place, zero incoming state
+  RowStream<double, P, M> L;
 #pragma unroll
-  for (int t = 1; t < M; ++t)
+  for (int t = 0; t < M; ++t) {
+    L.up(lo, t);
 #pragma unroll
     for (int i = 1; i <= P; ++i) {
       if (t - i < 0) continue;
-      const double l = tget(lo, t, i - 1);
+      const double l = L(t, i - 1);
 #pragma unroll
       for (int n = 0; n < NC; ++n) x[n][t] -= l * x[n][t - i];
     }
+  }
   op_fence();
   // carry: last P rows, c[q] = w_{r0+M-1-q}
   double c[NC][P];
@@ -250,8 +266,8 @@ __device__ __forceinline__ void lsolve(const TabRef lo, int lane, double (&x)[NC
       double acc = 0.0;
 #pragma unroll
       for (int i = 1; i <= P; ++i) {
-        if (t - i >= 0) acc -= tget(lo, t, i - 1) * g[t - i];
-        else if (i - t - 1 == b) acc -= tget(lo, t, i - 1);
+        if (t - i >= 0) acc -= L(t, i - 1) * g[t - i];
+        else if (i - t - 1 == b) acc -= L(t, i - 1);
       }
       g[t] = acc;
     }
@@ -271,14 +287,16 @@ __device__ __forceinline__ void lsolve(const TabRef lo, int lane, double (&x)[NC
       s[n][q] = lane == 0 ? 0.0 : v;
     }
   const TabRef lo2 = relaunder(lo);
+  RowStream<double, P, M> L2;
   double dl[NC][M];
 #pragma unroll
   for (int t = 0; t < M; ++t) {
+    L2.up(lo2, t);
 #pragma unroll
     for (int n = 0; n < NC; ++n) dl[n][t] = 0.0;
 #pragma unroll
     for (int i = 1; i <= P; ++i) {
-      const double l = tget(lo2, t, i - 1);
+      const double l = L2(t, i - 1);
 #pragma unroll
       for (int n = 0; n < NC; ++n) {
         const double pv = (t - i >= 0) ? dl[n][t - i] : s[n][i - t - 1];
@@ -291,19 +309,21 @@ __device__ __forceinline__ void lsolve(const TabRef lo, int lane, double (&x)[NC
 }
 
 // ---- upper solve: x_r = (w_r - sum_{d=1..P} U(r,d) x_{r+d}) * inv_r ------
+// up: rows of inv_r, U(r,1..P)
 template <int M, int P, int NC>
-__device__ __forceinline__ void usolve(const TabRef up, const TabRef inv, int lane,
-                                       double (&x)[NC][M]) {
+__device__ __forceinline__ void usolve(const TabRef up, int lane, double (&x)[NC][M]) {
+  RowStream<double, P + 1, M> U;
 #pragma unroll
   for (int t = M - 1; t >= 0; --t) {
+    U.down(up, t);
 #pragma unroll
     for (int d = 1; d <= P; ++d) {
       if (t + d >= M) continue;
-      const double u = tget(up, t, d - 1);
+      const double u = U(t, d);
 #pragma unroll
       for (int n = 0; n < NC; ++n) x[n][t] -= u * x[n][t + d];
     }
-    const double iv = tget(inv, t, 0);
+    const double iv = U(t, 0);
 #pragma unroll
     for (int n = 0; n < NC; ++n) x[n][t] *= iv;
   }
@@ -323,10 +343,10 @@ __device__ __forceinline__ void usolve(const TabRef up, const TabRef inv, int la
       double acc = 0.0;
 #pragma unroll
       for (int d = 1; d <= P; ++d) {
-        if (t + d < M) acc -= tget(up, t, d - 1) * g[t + d];
-        else if (t + d - M == b) acc -= tget(up, t, d - 1);
+        if (t + d < M) acc -= U(t, d) * g[t + d];
+        else if (t + d - M == b) acc -= U(t, d);
       }
-      g[t] = acc * tget(inv, t, 0);
+      g[t] = acc * U(t, 0);
     }
 #pragma unroll
     for (int q = 0; q < P; ++q) A[q][b] = g[q];
@@ -342,22 +362,24 @@ __device__ __forceinline__ void usolve(const TabRef up, const TabRef inv, int la
       const double v = __shfl_down(c[n][q], 1);
       s[n][q] = lane == WAVE - 1 ? 0.0 : v;
     }
-  const TabRef up2 = relaunder(up), inv2 = relaunder(inv);
+  const TabRef up2 = relaunder(up);
+  RowStream<double, P + 1, M> U2;
   double dl[NC][M];
 #pragma unroll
   for (int t = M - 1; t >= 0; --t) {
+    U2.down(up2, t);
 #pragma unroll
     for (int n = 0; n < NC; ++n) dl[n][t] = 0.0;
 #pragma unroll
     for (int d = 1; d <= P; ++d) {
-      const double u = tget(up2, t, d - 1);
+      const double u = U2(t, d);
 #pragma unroll
       for (int n = 0; n < NC; ++n) {
         const double pv = (t + d < M) ? dl[n][t + d] : s[n][t + d - M];
         dl[n][t] -= u * pv;
       }
     }
-    const double iv = tget(inv2, t, 0);
+    const double iv = U2(t, 0);
 #pragma unroll
     for (int n = 0; n < NC; ++n) {
       dl[n][t] *= iv;
@@ -369,23 +391,26 @@ __device__ __forceinline__ void usolve(const TabRef up, const TabRef inv, int la
 // ---- triangular solves with precomputed scan matrices -------------------
 // For a fixed factor the carry maps of the lanes do not depend on the data,
 // so the Hillis-Steele compositions are tabulated once per grid:
-// H[k][q][b][lane] (lane-major) is the map from the carry of lane l-2^k
-// (l+2^k for the upper solve) to that of lane l after the first k levels.
+// H[k] (a stream of P*P entries, q*P + b) is the map from the carry of lane
+// l-2^k (l+2^k for the upper solve) to that of lane l after k levels.
 // Only the first `levels` levels are applied: the compositions beyond them
 // are below 1e-22 in max norm (the factors' inverses decay geometrically),
 // checked when the tables are built.
 template <int M, int P, int NC, typename V>
 __device__ __forceinline__ void lsolve_tab(const TabRef lo, const TabRef H, int levels,
                                            int lane, V (&x)[NC][M]) {
+  RowStream<V, P, M> L;
 #pragma unroll
-  for (int t = 1; t < M; ++t)
+  for (int t = 1; t < M; ++t) {
+    L.up(lo, t, 1);
 #pragma unroll
     for (int i = 1; i <= P; ++i) {
       if (t - i < 0) continue;
-      const V l = tget_v<V>(lo, t, i - 1);
+      const V l = L(t, i - 1);
 #pragma unroll
       for (int n = 0; n < NC; ++n) x[n][t] -= l * x[n][t - i];
     }
+  }
   op_fence();
   V c[NC][P];
 #pragma unroll
@@ -398,12 +423,10 @@ __device__ __forceinline__ void lsolve_tab(const TabRef lo, const TabRef H, int 
       const int d = 1 << k;
       // the level's composed map is loaded before the shuffles and outside
       // the lane test, so its loads are in flight together
-      const TabRef Hk = relaunder_after(H, c[0][0]);
-      V h[P][P];
-#pragma unroll
-      for (int q = 0; q < P; ++q)
-#pragma unroll
-        for (int b = 0; b < P; ++b) h[q][b] = tget_v<V>(Hk, k * P + q, b);
+      TabRef Hk = relaunder_after(H, c[0][0]);
+      Hk.sbias += k * P * P * WAVE * (int)sizeof(V);
+      RowStream<V, P * P, 1> h;
+      h.up(Hk, 0);
       V cp[NC][P];
 #pragma unroll
       for (int n = 0; n < NC; ++n)
@@ -415,7 +438,7 @@ __device__ __forceinline__ void lsolve_tab(const TabRef lo, const TabRef H, int 
 #pragma unroll
           for (int b = 0; b < P; ++b)
 #pragma unroll
-            for (int n = 0; n < NC; ++n) c[n][q] += h[q][b] * cp[n][b];
+            for (int n = 0; n < NC; ++n) c[n][q] += h(0, q * P + b) * cp[n][b];
       }
     }
   }
@@ -429,14 +452,16 @@ __device__ __forceinline__ void lsolve_tab(const TabRef lo, const TabRef H, int 
       s[n][q] = lane == 0 ? V(0) : v;
     }
   const TabRef lo2 = relaunder(lo);
+  RowStream<V, P, M> L2;
   V dl[NC][M];
 #pragma unroll
   for (int t = 0; t < M; ++t) {
+    L2.up(lo2, t);
 #pragma unroll
     for (int n = 0; n < NC; ++n) dl[n][t] = V(0);
 #pragma unroll
     for (int i = 1; i <= P; ++i) {
-      const V l = tget_v<V>(lo2, t, i - 1);
+      const V l = L2(t, i - 1);
 #pragma unroll
       for (int n = 0; n < NC; ++n) {
         const V pv = (t - i >= 0) ? dl[n][t - i] : s[n][i - t - 1];
@@ -449,18 +474,20 @@ __device__ __forceinline__ void lsolve_tab(const TabRef lo, const TabRef H, int 
 }
 
 template <int M, int P, int NC, typename V>
-__device__ __forceinline__ void usolve_tab(const TabRef up, const TabRef inv, const TabRef H,
-                                           int levels, int lane, V (&x)[NC][M]) {
+__device__ __forceinline__ void usolve_tab(const TabRef up, const TabRef H, int levels,
+                                           int lane, V (&x)[NC][M]) {
+  RowStream<V, P + 1, M> U;
 #pragma unroll
   for (int t = M - 1; t >= 0; --t) {
+    U.down(up, t);
 #pragma unroll
     for (int d = 1; d <= P; ++d) {
       if (t + d >= M) continue;
-      const V u = tget_v<V>(up, t, d - 1);
+      const V u = U(t, d);
 #pragma unroll
       for (int n = 0; n < NC; ++n) x[n][t] -= u * x[n][t + d];
     }
-    const V iv = tget_v<V>(inv, t, 0);
+    const V iv = U(t, 0);
 #pragma unroll
     for (int n = 0; n < NC; ++n) x[n][t] *= iv;
   }
@@ -474,12 +501,10 @@ __device__ __forceinline__ void usolve_tab(const TabRef up, const TabRef inv, co
   for (int k = 0; k < 6; ++k) {
     if (k < levels) {
       const int d = 1 << k;
-      const TabRef Hk = relaunder_after(H, c[0][0]);
-      V h[P][P];
-#pragma unroll
-      for (int q = 0; q < P; ++q)
-#pragma unroll
-        for (int b = 0; b < P; ++b) h[q][b] = tget_v<V>(Hk, k * P + q, b);
+      TabRef Hk = relaunder_after(H, c[0][0]);
+      Hk.sbias += k * P * P * WAVE * (int)sizeof(V);
+      RowStream<V, P * P, 1> h;
+      h.up(Hk, 0);
       V cp[NC][P];
 #pragma unroll
       for (int n = 0; n < NC; ++n)
@@ -491,7 +516,7 @@ __device__ __forceinline__ void usolve_tab(const TabRef up, const TabRef inv, co
 #pragma unroll
           for (int b = 0; b < P; ++b)
 #pragma unroll
-            for (int n = 0; n < NC; ++n) c[n][q] += h[q][b] * cp[n][b];
+            for (int n = 0; n < NC; ++n) c[n][q] += h(0, q * P + b) * cp[n][b];
       }
     }
   }
@@ -504,22 +529,24 @@ __device__ __forceinline__ void usolve_tab(const TabRef up, const TabRef inv, co
       const V v = __shfl_down(c[n][q], 1);
       s[n][q] = lane == WAVE - 1 ? V(0) : v;
     }
-  const TabRef up2 = relaunder(up), inv2 = relaunder(inv);
+  const TabRef up2 = relaunder(up);
+  RowStream<V, P + 1, M> U2;
   V dl[NC][M];
 #pragma unroll
   for (int t = M - 1; t >= 0; --t) {
+    U2.down(up2, t);
 #pragma unroll
     for (int n = 0; n < NC; ++n) dl[n][t] = V(0);
 #pragma unroll
     for (int d = 1; d <= P; ++d) {
-      const V u = tget_v<V>(up2, t, d - 1);
+      const V u = U2(t, d);
 #pragma unroll
       for (int n = 0; n < NC; ++n) {
         const V pv = (t + d < M) ? dl[n][t + d] : s[n][t + d - M];
         dl[n][t] -= u * pv;
       }
     }
-    const V iv = tget_v<V>(inv2, t, 0);
+    const V iv = U2(t, 0);
 #pragma unroll
     for (int n = 0; n < NC; ++n) {
       dl[n][t] *= iv;
@@ -529,8 +556,8 @@ __device__ __forceinline__ void usolve_tab(const TabRef up, const TabRef inv, co
 }
 
 // ---- banded matvec y_r = sum_d B(r,d) u_{r-P+d} ---------------------------
-// ROWS: each row's coefficients are loaded together one row ahead
-// (row_ld / row_take); otherwise the scheduler places the loads.
+// ROWS: each row's coefficients are loaded together one row ahead and waited
+// for once; otherwise the scheduler places the loads.
 template <int M, int P, int NC, typename V, bool ROWS = true>
 __device__ __forceinline__ void bmatvec(const TabRef B, int lane, const V (&u)[NC][M],
                                         V (&y)[NC][M]) {
@@ -544,17 +571,16 @@ __device__ __forceinline__ void bmatvec(const TabRef B, int lane, const V (&u)[N
       hl[n][q] = lane == 0 ? V(0) : a;
       hr[n][q] = lane == WAVE - 1 ? V(0) : b;
     }
-  V bn[2 * P + 1];
-  if constexpr (ROWS) row_ld<2 * P + 1>(B, 0, bn);
+  RowStream<V, 2 * P + 1, M> bc;
+  if constexpr (ROWS) bc.up(B, 0);
 #pragma unroll
   for (int t = 0; t < M; ++t) {
-    V bc[2 * P + 1];
     if constexpr (ROWS) {
-      row_take<2 * P + 1>(bn, bc);
-      if (t + 1 < M) row_ld<2 * P + 1>(B, t + 1, bn);
+      bc.take(t);
+      if (t + 1 < M) bc.up(B, t + 1);
       op_fence();
     } else {
-      row_ld<2 * P + 1>(B, t, bc);
+      bc.up(B, t);
     }
     V acc[NC];
 #pragma unroll
@@ -562,7 +588,7 @@ __device__ __forceinline__ void bmatvec(const TabRef B, int lane, const V (&u)[N
 #pragma unroll
     for (int d = 0; d <= 2 * P; ++d) {
       const int col = t - P + d;
-      const V bv = bc[d];
+      const V bv = bc(t, d);
 #pragma unroll
       for (int n = 0; n < NC; ++n) {
         const V v = col < 0 ? hl[n][col + P] : (col >= M ? hr[n][col - M] : u[n][col]);
@@ -585,15 +611,15 @@ __device__ __forceinline__ double col_value(const double (&x)[M], int row) {
   return __shfl(mine, l);
 }
 
-// Tables of one y grid, in order, in one allocation.  Per-row tables hold
-// nb entries for each of 64*M rows (lane-major); the scan compositions of the
-// fixed factors hold 6 levels of P x P maps for 64 lanes.
+// Tables of one y grid, in order, in one allocation.  Per-row tables are
+// streams of M rows of ytab_width entries a lane; the scan compositions of
+// the fixed factors are 6 streams (levels) of one P x P map a lane.
 enum YTabId {
-  YT_B1, YT_A1, YT_INV1, YT_UP1, YT_LO1, YT_FMAP,  // d/deta: B1, A1, LU of A1, fmap
-  YT_B2, YT_A2, YT_INV2, YT_UP2, YT_LO2,           // d2/dy2: B2, A2, LU of A2
-  YT_INVI, YT_UPI, YT_LOI,                         // integration: LU of B1
-  YT_WBD,                                          // boundary d/dy functionals
-  YT_NROW,                                         // (count of per-row tables)
+  YT_B1, YT_A1, YT_U1, YT_LO1, YT_FMAP,  // d/deta: B1, A1, LU of A1 (U: inv, up), fmap
+  YT_B2, YT_A2, YT_U2, YT_LO2,           // d2/dy2: B2, A2, LU of A2
+  YT_UI, YT_LOI,                         // integration: LU of B1
+  YT_WBD,                                // boundary d/dy functionals
+  YT_NROW,                               // (count of per-row tables)
   YT_HL1 = YT_NROW, YT_HU1, YT_HL2, YT_HU2, YT_HLI, YT_HUI,
   YT_COUNT
 };
@@ -601,8 +627,9 @@ __host__ __device__ constexpr int ytab_width(int id) {
   // entries per row of the per-row tables; P of the scan tables
   return id == YT_B1 || id == YT_A1 ? 7
        : id == YT_B2 || id == YT_A2 ? 5
-       : id == YT_UP1 || id == YT_LO1 || id == YT_UPI || id == YT_LOI ? 3
-       : id == YT_UP2 || id == YT_LO2 || id == YT_WBD ? 2
+       : id == YT_U1 || id == YT_UI ? 4
+       : id == YT_LO1 || id == YT_LOI || id == YT_U2 ? 3
+       : id == YT_LO2 || id == YT_WBD ? 2
        : id == YT_HL1 || id == YT_HU1 || id == YT_HLI || id == YT_HUI ? 3
        : id == YT_HL2 || id == YT_HU2 ? 2 : 1;
 }
@@ -616,47 +643,41 @@ __host__ __device__ constexpr int ytab_offset(int id, int M) {
   return off;
 }
 
-// Device tables of one y grid: one allocation, lane-major tables of 64*M
-// rows each at the offsets ytab_offset(id, M) (loma_kernels.h), so that every
-// table access goes through one buffer resource with a constant offset.
+// Device tables of one y grid: one allocation, lane-major streams at the
+// offsets ytab_offset(id, M), so that every table access goes through one
+// buffer resource with a constant offset.
 struct YTab {
   const double* base;
-  const float* base32;  // the same tables rounded to FP32, same layout
+  const float* base32;  // the same tables rounded to FP32 (four to a vector)
   // scan level counts of the fixed factors (see lsolve_tab)
   int kL1, kU1, kL2, kU2, kLi, kUi;
   int my;
 };
 
-// view of table `id` (ncol entries per row) for this lane
-template <int M>
-__device__ __forceinline__ TabRef ytab(const YTab& T, int id, int ncol, int lane) {
-  return TabRef{make_rsrc(T.base, 0x7fffffff), ncol, 0, lane * 8, ytab_offset(id, M) * 8};
-}
-// ... in the arithmetic type V (read with tget_v<V>)
-template <int M, typename V>
-__device__ __forceinline__ TabRef ytab_v(const YTab& T, int id, int ncol, int lane) {
-  if constexpr (sizeof(V) == 8)
-    return ytab<M>(T, id, ncol, lane);
-  else
-    return TabRef{make_rsrc(T.base32, 0x7fffffff), ncol, 0, lane * 4, ytab_offset(id, M) * 4};
+// view of table `id` for this lane, in the arithmetic type V
+template <int M, typename V = double>
+__device__ __forceinline__ TabRef ytab(const YTab& T, int id, int lane) {
+  const void* base = T.base;
+  if constexpr (sizeof(V) == 4) base = T.base32;
+  return TabRef{make_rsrc(base, 0x7fffffff), lane * 16, ytab_offset(id, M) * (int)sizeof(V)};
 }
 
 // first derivative du = fmap * A1^{-1} B1 u   (deryr2, cfdiff.f:518-601)
 template <int M, int NC, typename V, bool ROWS = true>
 __device__ __forceinline__ void op_dy1(const YTab& T, int lane, const V (&u)[NC][M],
                                        V (&du)[NC][M], bool apply_fmap = true) {
-  bmatvec<M, 3, NC, V, ROWS>(ytab_v<M, V>(T, YT_B1, 7, lane), lane, u, du);
+  bmatvec<M, 3, NC, V, ROWS>(ytab<M, V>(T, YT_B1, lane), lane, u, du);
   op_fence();
-  lsolve_tab<M, 3, NC>(ytab_v<M, V>(T, YT_LO1, 3, lane), ytab_v<M, V>(T, YT_HL1, 3, lane), T.kL1, lane, du);
+  lsolve_tab<M, 3, NC>(ytab<M, V>(T, YT_LO1, lane), ytab<M, V>(T, YT_HL1, lane), T.kL1, lane, du);
   op_fence();
-  usolve_tab<M, 3, NC>(ytab_v<M, V>(T, YT_UP1, 3, lane), ytab_v<M, V>(T, YT_INV1, 1, lane),
-                       ytab_v<M, V>(T, YT_HU1, 3, lane), T.kU1, lane, du);
+  usolve_tab<M, 3, NC>(ytab<M, V>(T, YT_U1, lane), ytab<M, V>(T, YT_HU1, lane), T.kU1, lane, du);
   op_fence();
   if (apply_fmap) {
-    const TabRef fm = ytab_v<M, V>(T, YT_FMAP, 1, lane);
+    RowStream<V, 1, M> fm;
 #pragma unroll
     for (int t = 0; t < M; ++t) {
-      const V f = tget_v<V>(fm, t, 0);
+      fm.up(ytab<M, V>(T, YT_FMAP, lane), t);
+      const V f = fm(t, 0);
 #pragma unroll
       for (int n = 0; n < NC; ++n) du[n][t] *= f;
     }
@@ -668,24 +689,29 @@ __device__ __forceinline__ void op_dy1(const YTab& T, int lane, const V (&u)[NC]
 template <int M, int NC, typename V, bool ROWS = true>
 __device__ __forceinline__ void op_dy2(const YTab& T, int lane, const V (&u)[NC][M],
                                        V (&d2u)[NC][M]) {
-  bmatvec<M, 2, NC, V, ROWS>(ytab_v<M, V>(T, YT_B2, 5, lane), lane, u, d2u);
+  bmatvec<M, 2, NC, V, ROWS>(ytab<M, V>(T, YT_B2, lane), lane, u, d2u);
   op_fence();
-  lsolve_tab<M, 2, NC>(ytab_v<M, V>(T, YT_LO2, 2, lane), ytab_v<M, V>(T, YT_HL2, 2, lane), T.kL2, lane, d2u);
+  lsolve_tab<M, 2, NC>(ytab<M, V>(T, YT_LO2, lane), ytab<M, V>(T, YT_HL2, lane), T.kL2, lane, d2u);
   op_fence();
-  usolve_tab<M, 2, NC>(ytab_v<M, V>(T, YT_UP2, 2, lane), ytab_v<M, V>(T, YT_INV2, 1, lane),
-                       ytab_v<M, V>(T, YT_HU2, 2, lane), T.kU2, lane, d2u);
+  usolve_tab<M, 2, NC>(ytab<M, V>(T, YT_U2, lane), ytab<M, V>(T, YT_HU2, lane), T.kU2, lane, d2u);
   op_fence();
 }
 
 // Helmholtz/Poisson solve (dt22 - rK dt21) v = rhs with identity end rows,
-// LU per mode class in `lu` (lane-major, 5 entries per row: inv, up1, up2,
-// lo1, lo2), the RHS being dt21*f with zero end rows (calcrhslap,
+// LU per mode class in `lu` (a stream of rows lo1, lo2, then one of rows
+// inv, up1, up2), the RHS being dt21*f with zero end rows (calcrhslap,
 // laps.f:17-46).
+template <int M>
+__device__ __forceinline__ TabRef lu_lo(const double* lu, int lane) { return tab(lu, lane); }
+template <int M>
+__device__ __forceinline__ TabRef lu_up(const double* lu, int lane) {
+  return tab(lu + 2 * WAVE * M, lane);
+}
 template <int M, int NC>
 __device__ __forceinline__ void op_helm(const YTab& T, const double* __restrict__ lu,
                                         int lane, const double (&f)[NC][M],
                                         double (&v)[NC][M]) {
-  bmatvec<M, 2, NC, double, false>(ytab<M>(T, YT_A2, 5, lane), lane, f, v);
+  bmatvec<M, 2, NC, double, false>(ytab<M>(T, YT_A2, lane), lane, f, v);
   const int r0 = lane * M;
 #pragma unroll
   for (int t = 0; t < M; ++t) {
@@ -696,9 +722,9 @@ __device__ __forceinline__ void op_helm(const YTab& T, const double* __restrict_
     }
   }
   op_fence();
-  lsolve<M, 2, NC>(tab(lu, 5, 3, lane), lane, v);
+  lsolve<M, 2, NC>(lu_lo<M>(lu, lane), lane, v);
   op_fence();
-  usolve<M, 2, NC>(tab(lu, 5, 1, lane), tab(lu, 5, 0, lane), lane, v);
+  usolve<M, 2, NC>(lu_up<M>(lu, lane), lane, v);
   op_fence();
 }
 

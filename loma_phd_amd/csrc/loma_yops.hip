@@ -122,9 +122,9 @@ int launch_thickness(int M, bool fp32, const PhaseArgs& a, const double* hy, dou
 }
 
 // LU of (dt22 - s dt21) with identity end rows (Lapvdvhom laps.f:349-366),
-// one thread per shift s.  Output per class: a lane-major table of 64*M rows
-// with entries inv, up1, up2, lo1, lo2 (lower multipliers by destination
-// row), zero beyond row my-1.
+// one thread per shift s.  Output per class: lane-major streams over 64*M
+// rows, first lo1, lo2 (lower multipliers by destination row), then inv, up1,
+// up2; zero beyond row my-1.
 __global__ void k_helm_factor(const double* __restrict__ dt21,
                               const double* __restrict__ dt22, int my, int M,
                               const double* __restrict__ shifts, int nsys,
@@ -135,9 +135,11 @@ __global__ void k_helm_factor(const double* __restrict__ dt21,
   const int stride = 5 * WAVE * M;
   double* out = lu + (size_t)s * stride;
   for (int q = 0; q < stride; ++q) out[q] = 0.0;
+  // idx: 0 inv, 1 up1, 2 up2, 3 lo1, 4 lo2
   auto at = [&](int row, int idx) -> double& {
     const int l = row / M, t = row - l * M;
-    return out[(t * 5 + idx) * WAVE + l];
+    return idx < 3 ? out[2 * WAVE * M + stream_index(3 * M, t * 3 + idx, l, 2)]
+                   : out[stream_index(2 * M, t * 2 + idx - 3, l, 2)];
   };
   auto row = [&](int j, double* r) {
     if (j >= my) { for (int d = 0; d < 5; ++d) r[d] = 0.0; return; }

@@ -53,11 +53,12 @@ __device__ __forceinline__ double wave_sum(double v) {
 template <int M>
 __device__ __forceinline__ void bd_dots(const YTab& T, int lane, const double (&x)[2][M],
                                         double (&out)[4]) {
-  const TabRef w = ytab<M>(T, YT_WBD, 2, lane);
+  RowStream<double, 2, M> w;
   double s0r = 0.0, s0i = 0.0, s1r = 0.0, s1i = 0.0;
 #pragma unroll
   for (int t = 0; t < M; ++t) {
-    const double a = tget(w, t, 0), b = tget(w, t, 1);
+    w.up(ytab<M>(T, YT_WBD, lane), t);
+    const double a = w(t, 0), b = w(t, 1);
     s0r += a * x[0][t];
     s0i += a * x[1][t];
     s1r += b * x[0][t];
@@ -90,7 +91,7 @@ __device__ __forceinline__ void solve_neumann(const YTab& T, const double* lu,
   const double ci1 = (-dp[1] * a22 + a12 * dp[3]) / det;
   const double ci2 = (-a11 * dp[3] + a21 * dp[1]) / det;
   // second solve with Dirichlet end values (c1, c2)
-  bmatvec<M, 2, 2>(ytab<M>(T, YT_A2, 5, lane), lane, f, v);
+  bmatvec<M, 2, 2>(ytab<M>(T, YT_A2, lane), lane, f, v);
   const int r0 = lane * M;
 #pragma unroll
   for (int t = 0; t < M; ++t) {
@@ -98,8 +99,8 @@ __device__ __forceinline__ void solve_neumann(const YTab& T, const double* lu,
     if (r == 0) { v[0][t] = cr1; v[1][t] = ci1; }
     if (r == T.my - 1) { v[0][t] = cr2; v[1][t] = ci2; }
   }
-  lsolve<M, 2, 2>(tab(lu, 5, 3, lane), lane, v);
-  usolve<M, 2, 2>(tab(lu, 5, 1, lane), tab(lu, 5, 0, lane), lane, v);
+  lsolve<M, 2, 2>(lu_lo<M>(lu, lane), lane, v);
+  usolve<M, 2, 2>(lu_up<M>(lu, lane), lane, v);
 }
 
 // per-class Neumann constants: h1 = LU^{-1} e_0, h2 = LU^{-1} e_{my-1};
@@ -118,15 +119,15 @@ __global__ __launch_bounds__(256) void k_helm_bc(YTab T, const double* lu, int l
     h[0][t] = (r0 + t == 0) ? 1.0 : 0.0;
     h[1][t] = (r0 + t == T.my - 1) ? 1.0 : 0.0;
   }
-  lsolve<M, 2, 2>(tab(L, 5, 3, lane), lane, h);
-  usolve<M, 2, 2>(tab(L, 5, 1, lane), tab(L, 5, 0, lane), lane, h);
+  lsolve<M, 2, 2>(lu_lo<M>(L, lane), lane, h);
+  usolve<M, 2, 2>(lu_up<M>(L, lane), lane, h);
   if (hout) {
-    // h1, h2 lane-major (entry 0: h1, entry 1: h2 of row lane*M + t)
+    // a stream of rows h1, h2
     double* H = hout + (size_t)wave * 2 * WAVE * M;
 #pragma unroll
     for (int t = 0; t < M; ++t) {
-      H[(t * 2 + 0) * WAVE + lane] = h[0][t];
-      H[(t * 2 + 1) * WAVE + lane] = h[1][t];
+      H[stream_index(2 * M, t * 2 + 0, lane, 2)] = h[0][t];
+      H[stream_index(2 * M, t * 2 + 1, lane, 2)] = h[1][t];
     }
   }
   double d[4];
@@ -272,15 +273,15 @@ __global__ __launch_bounds__(256) void k_visc(YTab T, const double* lu1, const d
     const double c3i = (dp[1] * m22 + m12 * dp[3]) / det;
     const double c4i = (-m11 * dp[3] - m21 * dp[1]) / det;
     // second Dirichlet solve with end values (c3, c4)
-    bmatvec<M, 2, 2>(ytab<M>(T, YT_A2, 5, lane), lane, x, vp);
+    bmatvec<M, 2, 2>(ytab<M>(T, YT_A2, lane), lane, x, vp);
 #pragma unroll
     for (int t = 0; t < M; ++t) {
       const int r = r0 + t;
       if (r == 0) { vp[0][t] = c3r; vp[1][t] = c3i; }
       if (r == my - 1) { vp[0][t] = c4r; vp[1][t] = c4i; }
     }
-    lsolve<M, 2, 2>(tab(L2, 5, 3, lane), lane, vp);
-    usolve<M, 2, 2>(tab(L2, 5, 1, lane), tab(L2, 5, 0, lane), lane, vp);
+    lsolve<M, 2, 2>(lu_lo<M>(L2, lane), lane, vp);
+    usolve<M, 2, 2>(lu_up<M>(L2, lane), lane, vp);
     store_col<M>(v + o, my, lane, st, vp);
     op_dy1<M, 2>(T, lane, vp, f);
     store_col<M>(dvdy + o, my, lane, st, f);
@@ -295,17 +296,18 @@ template <int M>
 __device__ __forceinline__ void op_inty(const YTab& T, int lane, double (&x)[1][M]) {
   double f[1][M];
   const int r0 = lane * M;
-  const TabRef fm = ytab<M>(T, YT_FMAP, 1, lane);
+  RowStream<double, 1, M> fm;
 #pragma unroll
-  for (int t = 0; t < M; ++t) f[0][t] = (r0 + t < T.my) ? x[0][t] / tget(fm, t, 0) : 0.0;
-  bmatvec<M, 3, 1>(ytab<M>(T, YT_A1, 7, lane), lane, f, x);
+  for (int t = 0; t < M; ++t) {
+    fm.up(ytab<M>(T, YT_FMAP, lane), t);
+    f[0][t] = (r0 + t < T.my) ? x[0][t] / fm(t, 0) : 0.0;
+  }
+  bmatvec<M, 3, 1>(ytab<M>(T, YT_A1, lane), lane, f, x);
 #pragma unroll
   for (int t = 0; t < M; ++t)
     if (r0 + t == T.my - 1) x[0][t] = 0.0;  // gauge row x(my) = 0
-  lsolve_tab<M, 3, 1>(ytab<M>(T, YT_LOI, 3, lane), ytab<M>(T, YT_HLI, 3, lane), T.kLi, lane, x);
-  usolve_tab<M, 3, 1>(ytab<M>(T, YT_UPI, 3, lane), ytab<M>(T, YT_INVI, 1, lane),
-                      ytab<M>(T, YT_HUI, 3, lane),
-                      T.kUi, lane, x);
+  lsolve_tab<M, 3, 1>(ytab<M>(T, YT_LOI, lane), ytab<M>(T, YT_HLI, lane), T.kLi, lane, x);
+  usolve_tab<M, 3, 1>(ytab<M>(T, YT_UI, lane), ytab<M>(T, YT_HUI, lane), T.kUi, lane, x);
   const double v0 = col_value<M>(x[0], 0);
 #pragma unroll
   for (int t = 0; t < M; ++t) x[0][t] -= v0;
@@ -515,13 +517,14 @@ __global__ __launch_bounds__(256, 3) void k_phaseC32_batch(const PhaseArgs* __re
 template <int M>
 __device__ __forceinline__ void bd_dots4(const YTab& T, int lane, const double (&x)[4][M],
                                          double (&out)[8]) {
-  const TabRef w = ytab<M>(T, YT_WBD, 2, lane);
+  RowStream<double, 2, M> w;
   double s[8];
 #pragma unroll
   for (int q = 0; q < 8; ++q) s[q] = 0.0;
 #pragma unroll
   for (int t = 0; t < M; ++t) {
-    const double a = tget(w, t, 0), b = tget(w, t, 1);
+    w.up(ytab<M>(T, YT_WBD, lane), t);
+    const double a = w(t, 0), b = w(t, 1);
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
       s[n] += a * x[n][t];
