@@ -951,6 +951,7 @@ static FftArgs fft_args(loma_run* r, int rkstep, int do_cfl) {
   a.with_z = r->with_z ? 1 : 0;
   a.J = r->J;
   a.L = r->L;
+  a.xrow = xrow_serves(r->fp32, a) ? 1 : 0;
   return a;
 }
 
@@ -1137,12 +1138,12 @@ static int ens_batch_env() {
 
 static void ensemble_plan(loma_run* const* runs, int nruns, const std::vector<int>& icfl,
                           int cap, EnsPlan& plan) {
-  std::vector<std::array<int, 7>> keys;
+  std::vector<std::array<int, 8>> keys;
   std::vector<std::vector<int>> groups;
   for (int q = 0; q < nruns; ++q) {
     loma_run* r = runs[q];
-    const std::array<int, 7> k{r->M, r->fp32 ? 1 : 0, r->mgalz, r->J, r->mgalx, r->L,
-                               r->with_z ? 1 : 0};
+    const std::array<int, 8> k{r->M, r->fp32 ? 1 : 0, r->mgalz, r->J, r->mgalx, r->L,
+                               r->with_z ? 1 : 0, fft_args(r, 1, 0).xrow};
     size_t c = 0;
     while (c < keys.size() && keys[c] != k) ++c;
     if (c == keys.size()) { keys.push_back(k); groups.emplace_back(); }

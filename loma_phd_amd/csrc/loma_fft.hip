@@ -100,6 +100,20 @@ __device__ __forceinline__ void dft3(T2* v, int s) {
   v[2] = csub(m, r);
 }
 template <typename T, typename T2>
+__device__ __forceinline__ void dft6(T2* v, int s) {
+  T2 e[3] = {v[0], v[2], v[4]}, o[3] = {v[1], v[3], v[5]};
+  dft3<T, T2>(e, s);
+  dft3<T, T2>(o, s);
+  const T c = (T)0.5, h = (T)(0.86602540378443864676) * (T)s;
+  const T2 o1 = cmul(o[1], T2{c, h}), o2 = cmul(o[2], T2{-c, h});  // exp(s i pi k/3)
+  v[0] = cadd(e[0], o[0]);
+  v[3] = csub(e[0], o[0]);
+  v[1] = cadd(e[1], o1);
+  v[4] = csub(e[1], o1);
+  v[2] = cadd(e[2], o2);
+  v[5] = csub(e[2], o2);
+}
+template <typename T, typename T2>
 __device__ __forceinline__ void dft5(T2* v, int s) {
   const T c1 = (T)0.30901699437494742410, c2 = (T)-0.80901699437494742410;
   const T s1 = (T)0.95105651629515357212 * (T)s, s2 = (T)0.58778525229247312917 * (T)s;
@@ -167,8 +181,8 @@ __device__ __forceinline__ void twiddle_pow(T2* w, T2 p1, int s) {
   if constexpr (R >= 3) p[2] = cmul(p[1], p[1]);
   if constexpr (R >= 4) p[3] = cmul(p[2], p[1]);
   if constexpr (R >= 5) p[4] = cmul(p[2], p[2]);
+  if constexpr (R >= 6) p[5] = cmul(p[4], p[1]);
   if constexpr (R >= 8) {
-    p[5] = cmul(p[4], p[1]);
     p[6] = cmul(p[3], p[3]);
     p[7] = cmul(p[4], p[3]);
   }
@@ -209,34 +223,12 @@ __device__ __forceinline__ void stockham_item(const T2* __restrict__ src, T2* __
   for (int r = 0; r < R; ++r) dst[lds_i<PAD>(idxD + r * Ns)] = v[r];
 }
 
-// The same butterfly with its first twiddle p1 = tw[(j % Ns) * tstep]
-// already in a register (no global load inside the pass)
-template <int R, typename T, typename T2, int PAD = LOMA_LDS_PAD>
-__device__ __forceinline__ void stockham_item_p1(const T2* __restrict__ src,
-                                                 T2* __restrict__ dst, int rowbase, int j,
-                                                 int nb, int Ns, T2 p1, int s) {
-  static_assert(LOMA_TW_REC, "register twiddles are the first power only");
-  T2 v[R];
-  const int jm = j % Ns;
-#pragma unroll
-  for (int r = 0; r < R; ++r) v[r] = src[lds_i<PAD>(rowbase + j + r * nb)];
-  if (Ns > 1) twiddle_pow<R>(v, p1, s);
-  if (R == 2) dft2<T, T2>(v);
-  if (R == 3) dft3<T, T2>(v, s);
-  if (R == 4) dft4<T, T2>(v, s);
-  if (R == 5) dft5<T, T2>(v, s);
-  if (R == 8) dft8<T, T2>(v, s);
-  const int idxD = rowbase + (j / Ns) * Ns * R + jm;
-#pragma unroll
-  for (int r = 0; r < R; ++r) dst[lds_i<PAD>(idxD + r * Ns)] = v[r];
-}
-
 // nrows independent length-N transforms of rows stored with stride N in a
 // (LDS, padded layout lds_i); b is scratch of the same size.  Returns the
 // buffer holding the result.  s = -1 forward (e^{-i}), +1 inverse; unscaled.
 // Ends with a barrier.
 template <typename T, typename T2, int PAD = LOMA_LDS_PAD>
-__device__ T2* fft_rows(T2* a, T2* b, int N, int RS, int nrows, const FftPlan& pl,
+__device__ __forceinline__ T2* fft_rows(T2* a, T2* b, int N, int RS, int nrows, const FftPlan& pl,
                         const T2* __restrict__ tw, int s) {
   int Ns = 1;
   for (int p = 0; p < pl.npass; ++p) {
@@ -332,48 +324,6 @@ constexpr int ct_radix(int m) {
   return m % 8 == 0 ? 8 : (m % 4 == 0 ? 4 : (m % 2 == 0 ? 2 : (m % 3 == 0 ? 3 : 5)));
 }
 
-// WR: every pass has 64 items per row (length 512 in radix 8), so the items
-// of a row stay in one wavefront from pass to pass; the passes are then
-// separated by wavefront barriers and only the last ends with a workgroup
-// barrier (its result is read across waves).
-#ifndef LOMA_XL_WR
-#define LOMA_XL_WR 1
-#endif
-// TWR (with WR, N = 512): the first twiddles of the passes come from a
-// copy in LDS, twl[j] = tw[j] (Ns = 64) and twl[64 + j % 8] = tw[(j % 8) * 8]
-// (Ns = 8); the passes then issue no global loads, so they do not wait
-// (vmcnt counts loads and stores in order) for the previous field's stores.
-template <typename T, typename T2, int N, int Ns, int NT, int RS, int PAD = LOMA_LDS_PAD,
-          bool WR = false, bool TWR = false>
-__device__ __forceinline__ T2* fft_rows_ct(T2* a, T2* b, int nrows, const T2* __restrict__ tw,
-                                           int s, const T2* twl = nullptr) {
-  if constexpr (Ns >= N) {
-    return a;
-  } else {
-    constexpr int R = ct_radix(N / Ns);
-    constexpr int nb = N / R;
-    constexpr int tstep = N / (Ns * R);
-    static_assert(!TWR || (WR && N == 512 && R == 8), "register twiddles: 512 = 8 x 8 x 8");
-    // the pass's index arithmetic starts here, not hoisted into earlier
-    // passes where it would hold registers across them
-    int t0 = threadIdx.x;
-    asm volatile("" : "+v"(t0));
-    const int total = nrows * nb;
-    for (int it = t0; it < total; it += NT) {
-      const int row = it / nb, j = it - row * nb;
-      if constexpr (TWR)
-        stockham_item_p1<R, T, T2, PAD>(a, b, row * RS, j, nb, Ns,
-                                        Ns == 8 ? twl[64 + (j & 7)] : twl[j], s);
-      else
-        stockham_item<R, T, T2, PAD>(a, b, row * RS, j, nb, Ns, tstep, tw, s);
-    }
-    static_assert(!WR || (nb == 64 && NT % 64 == 0), "wave-local rows need 64 items per row");
-    if constexpr (WR && Ns * R < N) wave_sync();
-    else __syncthreads();
-    return fft_rows_ct<T, T2, N, Ns * R, NT, RS, PAD, WR, TWR>(b, a, nrows, tw, s, twl);
-  }
-}
-
 template <typename T, typename T2, int E, int N, int Ns, int NT, int PAD, int NSTOP = N>
 __device__ __forceinline__ void fft_rows_ip_ct(T2* a, int nrows, const T2* __restrict__ tw,
                                                int s, T2* v) {
@@ -431,30 +381,11 @@ __device__ __forceinline__ void dft_r(T2* w, int s) {
   if constexpr (R == 3) dft3<T, T2>(w, s);
   if constexpr (R == 4) dft4<T, T2>(w, s);
   if constexpr (R == 5) dft5<T, T2>(w, s);
+  if constexpr (R == 6) dft6<T, T2>(w, s);
   if constexpr (R == 8) dft8<T, T2>(w, s);
 }
 
 // NN > 0: compile-time length NN; NN = 0: the run-time plan
-// LOMA_XL_RS1 = 1 stores x-line rows with an odd stride (in entries); it
-// was measured slower than the even stride at 512x513x256, so it is off
-#ifndef LOMA_XL_RS1
-#define LOMA_XL_RS1 0
-#endif
-template <int NN>
-__device__ __forceinline__ int xl_row_stride(int N) { return (NN ? NN : N) + LOMA_XL_RS1; }
-
-// TWR: the 512-point plan's first twiddles from the LDS copy twl
-// (fft_rows_ct)
-template <typename T, typename T2, int NN, int NT, int PAD = LOMA_LDS_PAD, bool TWR = false>
-__device__ __forceinline__ T2* fft_any(T2* a, T2* b, int N, int nrows, const FftPlan& pl,
-                                       const T2* __restrict__ tw, int s,
-                                       const T2* twl = nullptr) {
-  if constexpr (NN > 0)
-    return fft_rows_ct<T, T2, NN, 1, NT, NN + LOMA_XL_RS1, PAD,
-                       (NN == 512 && LOMA_XL_WR != 0), TWR>(a, b, nrows, tw, s, twl);
-  else
-    return fft_rows<T, T2, PAD>(a, b, N, N + LOMA_XL_RS1, nrows, pl, tw, s);
-}
 template <typename T, typename T2, int E, int NN, int NT, int PAD>
 __device__ __forceinline__ void fft_any_ip(T2* a, int N, int nrows, const FftPlan& pl,
                                            const T2* __restrict__ tw, int s) {
@@ -646,19 +577,16 @@ __device__ __forceinline__ int xcd_tile(int b, int n) {
 __host__ inline int xcd_groups(int n) { return 8 * ((n + 7) / 8); }
 
 // Per-thread share of one input field's lines: XR (kx, line pair) items of
-// two complex coefficients, all loaded before the first is packed.  The
-// FP32 512-point path fetches the next field's share while the current one
-// is transformed (LOMA_XL_PF); elsewhere the held registers cost more than
-// the hidden latency (FP32 at 3 waves per SIMD) or gained nothing (FP64).
+// two complex coefficients, all loaded before the first is packed.
 template <typename T2, int XR>
 struct XlIn {
   T2 a[XR], b[XR];
 };
 
-template <typename T2, int XR, int NN>
+template <typename T2, int XR>
 __device__ __forceinline__ void xl_fetch(const FftArgs& a, const T2* __restrict__ src, int z,
                                          int j0, int pairs, XlIn<T2, XR>& v) {
-  const int np = NN ? NN / 3 : a.rc.nplanes, my = a.rc.my, mgz = a.rc.mgalz;
+  const int np = a.rc.nplanes, my = a.rc.my, mgz = a.rc.mgalz;
   const int lp = __builtin_ctz(pairs);  // pairs is a power of two
 #pragma unroll
   for (int r = 0; r < XR; ++r) {
@@ -709,13 +637,13 @@ constexpr int xl_pad() {
 
 // fetched lines of NF fields (xl_fetch) -> Hermitian-packed complex rows in
 // A (row f*pairs + p = lines j0+2p, j0+2p+1 of field f); no barrier.
-template <typename T, typename T2, int XR, int NN, int NF>
+template <typename T, typename T2, int XR, int NF>
 __device__ __forceinline__ void xl_pack_from(const FftArgs& a, const XlIn<T2, XR>* v, T2* A,
                                              int pairs) {
   constexpr int XP = xl_pad<T>();
-  const int N = NN ? NN : a.rc.mgalx, np = NN ? NN / 3 : a.rc.nplanes;
+  const int N = a.rc.mgalx, np = a.rc.nplanes;
   const int lp = __builtin_ctz(pairs);
-  const int RS = xl_row_stride<NN>(N);
+  const int RS = N;
   // the dealiased band np..N-np is zero
   const int nzero = N - 2 * np + 1;
   for (int it = threadIdx.x; it < NF * pairs * nzero; it += XL_THREADS) {
@@ -744,26 +672,25 @@ __device__ __forceinline__ void xl_pack_from(const FftArgs& a, const XlIn<T2, XR
 }
 // lines of NF fields (W layout [i][z][j]; src1 unused for NF = 1) -> the
 // packed rows in A; no barrier.
-template <typename T, typename T2, int XR, int NN, int NF>
+template <typename T, typename T2, int XR, int NF>
 __device__ __forceinline__ void xl_pack(const FftArgs& a, const T2* __restrict__ src0,
                                         const T2* __restrict__ src1, T2* A, int z, int j0,
                                         int pairs) {
   XlIn<T2, XR> v[NF];
-  xl_fetch<T2, XR, NN>(a, src0, z, j0, pairs, v[0]);
-  if constexpr (NF > 1) xl_fetch<T2, XR, NN>(a, src1, z, j0, pairs, v[1]);
-  xl_pack_from<T, T2, XR, NN, NF>(a, v, A, pairs);
+  xl_fetch<T2, XR>(a, src0, z, j0, pairs, v[0]);
+  if constexpr (NF > 1) xl_fetch<T2, XR>(a, src1, z, j0, pairs, v[1]);
+  xl_pack_from<T, T2, XR, NF>(a, v, A, pairs);
 }
 
 // Hermitian unpacking of the transformed pairs in R into fields dst0 (rows
 // 0..pairs-1) and dst1 (rows pairs..2*pairs-1), scaled by 1/N; no barrier.
-template <typename T, typename T2, int NN, int NF>
+template <typename T, typename T2, int NF>
 __device__ __forceinline__ void xl_unpack(const FftArgs& a, const T2* R, T2* __restrict__ dst0,
                                           T2* __restrict__ dst1, int z, int j0, int pairs) {
   constexpr int XP = xl_pad<T>();
-  const int N = NN ? NN : a.rc.mgalx, np = NN ? NN / 3 : a.rc.nplanes, my = a.rc.my,
-            mgz = a.rc.mgalz;
+  const int N = a.rc.mgalx, np = a.rc.nplanes, my = a.rc.my, mgz = a.rc.mgalz;
   const int lp = __builtin_ctz(pairs);
-  const int RS = xl_row_stride<NN>(N);
+  const int RS = N;
   const T hs = (T)(0.5 / (double)N);
   const int per = np * pairs;
   for (int it = threadIdx.x; it < NF * per; it += XL_THREADS) {
@@ -784,228 +711,26 @@ __device__ __forceinline__ void xl_unpack(const FftArgs& a, const T2* R, T2* __r
   }
 }
 
-// first twiddles of the 512-point passes (radix 8, 8, 8) for lane j:
-// tw[(j % 8) * 8] (the Ns = 8 pass) and tw[j] (Ns = 64)
-template <typename T2>
-struct XlTw {
-  T2 w8, w64;
-};
-template <typename T2>
-__device__ __forceinline__ XlTw<T2> xl_tw(const FftArgs& a) {
-  const T2* tw = (const T2*)a.twx;
-  const int j = threadIdx.x & 63;
-  return XlTw<T2>{tw[(j & 7) * 8], tw[j]};
-}
-// LOMA_XL_TWR = 1: the 512-point x lines outside the register-resident path
-// (FP64) take those twiddles from a 72-entry LDS copy (fft_rows_ct's TWR;
-// in registers they held 8 VGPRs across the kernel and made it spill)
-#ifndef LOMA_XL_TWR
-#define LOMA_XL_TWR 1
-#endif
-
 // pack, then the inverse FFT.  Returns the buffer holding the physical pairs.
-// TWR: the 512-point plan's first twiddles from the 72-entry LDS copy twl;
-// TWF: every twiddle from twl holding the whole table (other lengths)
-template <typename T, typename T2, int XR, int NN, int NF, bool TWR = false, bool TWF = false>
+template <typename T, typename T2, int XR, int NF>
 __device__ __forceinline__ T2* xl_inverse(const FftArgs& a, const T2* __restrict__ src0,
-                          const T2* __restrict__ src1, T2* A, T2* B, int z, int j0, int pairs,
-                          const T2* twl = nullptr) {
-  xl_pack<T, T2, XR, NN, NF>(a, src0, src1, A, z, j0, pairs);
+                          const T2* __restrict__ src1, T2* A, T2* B, int z, int j0, int pairs) {
+  xl_pack<T, T2, XR, NF>(a, src0, src1, A, z, j0, pairs);
   __syncthreads();
-  const int N = NN ? NN : a.rc.mgalx;
-  const T2* tw = TWF ? twl : (const T2*)a.twx;
-  return fft_any<T, T2, NN, XL_THREADS, xl_pad<T>(), TWR>(A, B, N, NF * pairs, a.plx, tw, +1,
-                                                           twl);
+  const int N = a.rc.mgalx;
+  return fft_rows<T, T2, xl_pad<T>()>(A, B, N, N, NF * pairs, a.plx, (const T2*)a.twx, +1);
 }
 
 // forward FFT of A (rows of NF outputs, filled by the caller, then
 // synchronised here) and the unpacking
-template <typename T, typename T2, int NN, int NF, bool TWR = false, bool TWF = false>
+template <typename T, typename T2, int NF>
 __device__ __forceinline__ void xl_forward(const FftArgs& a, T2* __restrict__ dst0, T2* __restrict__ dst1,
-                           T2* A, T2* B, int z, int j0, int pairs, const T2* twl = nullptr) {
-  const int N = NN ? NN : a.rc.mgalx;
+                           T2* A, T2* B, int z, int j0, int pairs) {
+  const int N = a.rc.mgalx;
   __syncthreads();
-  const T2* tw = TWF ? twl : (const T2*)a.twx;
-  const T2* R = fft_any<T, T2, NN, XL_THREADS, xl_pad<T>(), TWR>(A, B, N, NF * pairs, a.plx,
-                                                                  tw, -1, twl);
-  xl_unpack<T, T2, NN, NF>(a, R, dst0, dst1, z, j0, pairs);
+  const T2* R = fft_rows<T, T2, xl_pad<T>()>(A, B, N, N, NF * pairs, a.plx, (const T2*)a.twx, -1);
+  xl_unpack<T, T2, NF>(a, R, dst0, dst1, z, j0, pairs);
   __syncthreads();
-}
-
-// Register-resident ends of the 512-point transform (radix 8, 8, 8) for 4
-// pairs (4 rows, 256 items per pass: one per thread, row tid/64, item
-// j = tid%64).  The last inverse pass reads and writes entries j + 64r of its
-// row, which are exactly the entries x0 + 64m the physics assigns to the
-// thread; so the inverse keeps its last pass in registers (no store, no
-// barrier, no reload) and the forward takes its first pass from registers.
-// Barriers of the register-resident path.  Its radix passes are local to a
-// wavefront (wave p owns line pair p), so LOMA_XL_WAVE = 2 (default) puts
-// only a wavefront barrier between them and keeps workgroup barriers around
-// the pack and unpack, whose coalesced lane mapping crosses waves: 2.74
-// against 2.77 ms per launch at 512x513x256.  LOMA_XL_WAVE = 1 also packs
-// and unpacks per wave (16 bytes per lane instead of 64-byte runs, no
-// workgroup barrier at all): 2.80 ms.  0: workgroup barriers throughout.
-#ifndef LOMA_XL_WAVE
-#define LOMA_XL_WAVE 2
-#endif
-// barrier between two wave-local steps (LOMA_XL_WAVE >= 1: the lanes of
-// one wavefront only) and between steps that cross waves (a workgroup
-// barrier unless everything is wave-local, LOMA_XL_WAVE = 1)
-template <typename T, typename T2>
-__device__ __forceinline__ void xl_sync() {
-  if constexpr (LOMA_XL_WAVE >= 1) wave_sync();
-  else __syncthreads();
-}
-template <typename T, typename T2>
-__device__ __forceinline__ void xl_sync_x() {
-  if constexpr (LOMA_XL_WAVE == 1) wave_sync();
-  else __syncthreads();
-}
-
-// LOMA_XL_PF = 1: the register-resident path takes the first twiddles of
-// its passes from registers (loaded once per workgroup) and fetches the next
-// input field while the current one is transformed.  vmcnt counts loads and
-// stores in order, so a twiddle load inside a pass would make the pass wait
-// for the prefetch (and for the previous field's stores).
-#ifndef LOMA_XL_PF
-#define LOMA_XL_PF 1
-#endif
-static_assert(!LOMA_XL_PF || LOMA_XL_WAVE == 2, "the prefetch feeds the workgroup pack");
-// inverse transform of a fetched field (LOMA_XL_PF)
-template <typename T, typename T2, int XR>
-__device__ __forceinline__ void xl_inverse_reg_in(const FftArgs& a, const XlIn<T2, XR>& in,
-                                                  T2* A, T2* B, int pairs, const XlTw<T2>& tw,
-                                                  T (&v)[8][2]) {
-  constexpr int RS = 512 + LOMA_XL_RS1;
-  const int row = threadIdx.x >> 6, j = threadIdx.x & 63;
-  xl_pack_from<T, T2, XR, 512, 1>(a, &in, A, pairs);
-  xl_sync_x<T, T2>();
-  stockham_item_p1<8, T, T2, 0>(A, B, row * RS, j, 64, 1, tw.w8, +1);  // Ns = 1: no twiddles
-  xl_sync<T, T2>();
-  stockham_item_p1<8, T, T2, 0>(B, A, row * RS, j, 64, 8, tw.w8, +1);
-  xl_sync<T, T2>();
-  T2 w[8];
-#pragma unroll
-  for (int r = 0; r < 8; ++r) w[r] = A[row * RS + j + r * 64];
-  twiddle_pow<8>(w, tw.w64, +1);
-  dft8<T, T2>(w, +1);
-#pragma unroll
-  for (int r = 0; r < 8; ++r) {
-    v[r][0] = w[r].x;
-    v[r][1] = w[r].y;
-  }
-  xl_sync_x<T, T2>();  // A is packed again by the next field
-}
-
-template <typename T, typename T2, int XR>
-__device__ __forceinline__ void xl_inverse_reg(const FftArgs& a, const T2* __restrict__ src,
-                                               T2* A, T2* B, int z, int j0, int pairs,
-                                               T (&v)[8][2]) {
-  static_assert(xl_pad<T>() == 0, "register ends assume unpadded rows");
-  constexpr int RS = 512 + LOMA_XL_RS1;
-  const T2* tw = (const T2*)a.twx;
-  const int row = threadIdx.x >> 6, j = threadIdx.x & 63;
-  if constexpr (LOMA_XL_WAVE == 1) {
-    // wave `row` packs line pair `row`: lane j takes coefficients ii = j + 64k
-    constexpr int np = 512 / 3;
-    const int ja = j0 + 2 * row, jb = ja + 1, my = a.rc.my, mgz = a.rc.mgalz;
-    T2* Ar = A + row * RS;
-    T2 ca[3], cb[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const int ii = j + 64 * k;
-      ca[k] = T2{0, 0};
-      cb[k] = T2{0, 0};
-      if (ii < np) {
-        const size_t base = ((size_t)ii * mgz + z) * a.rc.myp;
-        if (ja < my) ca[k] = src[base + ja];
-        if (jb < my) cb[k] = src[base + jb];
-      }
-    }
-    for (int q = j; q < 512 - 2 * np + 1; q += 64) Ar[np + q] = T2{0, 0};  // dealiased band
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const int ii = j + 64 * k;
-      if (ii < np) {
-        if (ii == 0) {
-          Ar[0] = T2{ca[k].x, cb[k].x};  // kx = 0: imaginary part ignored (rftsingle.f:87-91)
-        } else {
-          Ar[ii] = T2{ca[k].x - cb[k].y, ca[k].y + cb[k].x};
-          Ar[512 - ii] = T2{ca[k].x + cb[k].y, -ca[k].y + cb[k].x};
-        }
-      }
-    }
-  } else {
-    xl_pack<T, T2, XR, 512, 1>(a, src, nullptr, A, z, j0, pairs);
-  }
-  xl_sync_x<T, T2>();
-  stockham_item<8, T, T2, 0>(A, B, row * RS, j, 64, 1, 64, tw, +1);
-  xl_sync<T, T2>();
-  stockham_item<8, T, T2, 0>(B, A, row * RS, j, 64, 8, 8, tw, +1);
-  xl_sync<T, T2>();
-  T2 w[8];
-#pragma unroll
-  for (int r = 0; r < 8; ++r) w[r] = A[row * RS + j + r * 64];
-  twiddle<8>(w, tw, j, 1, +1);
-  dft8<T, T2>(w, +1);
-#pragma unroll
-  for (int r = 0; r < 8; ++r) {
-    v[r][0] = w[r].x;
-    v[r][1] = w[r].y;
-  }
-  xl_sync_x<T, T2>();  // A is packed again by the next field
-}
-
-template <typename T, typename T2, bool PF>
-__device__ __forceinline__ void xl_forward_reg(const FftArgs& a, T2* __restrict__ dst, T2* A,
-                                               T2* B, int z, int j0, int pairs,
-                                               const T (&v)[8][2], const XlTw<T2>& twr) {
-  static_assert(xl_pad<T>() == 0, "register ends assume unpadded rows");
-  constexpr int RS = 512 + LOMA_XL_RS1;
-  const T2* tw = (const T2*)a.twx;
-  const int row = threadIdx.x >> 6, j = threadIdx.x & 63;
-  T2 w[8];
-#pragma unroll
-  for (int r = 0; r < 8; ++r) w[r] = T2{v[r][0], v[r][1]};
-  dft8<T, T2>(w, -1);  // first pass (no twiddles): entries j + 64r -> 8j + r
-#pragma unroll
-  for (int r = 0; r < 8; ++r) A[row * RS + 8 * j + r] = w[r];
-  xl_sync<T, T2>();
-  if constexpr (PF) {
-    stockham_item_p1<8, T, T2, 0>(A, B, row * RS, j, 64, 8, twr.w8, -1);
-    xl_sync<T, T2>();
-    stockham_item_p1<8, T, T2, 0>(B, A, row * RS, j, 64, 64, twr.w64, -1);
-  } else {
-    stockham_item<8, T, T2, 0>(A, B, row * RS, j, 64, 8, 8, tw, -1);
-    xl_sync<T, T2>();
-    stockham_item<8, T, T2, 0>(B, A, row * RS, j, 64, 64, 1, tw, -1);
-  }
-  xl_sync_x<T, T2>();
-  if constexpr (LOMA_XL_WAVE == 1) {
-    // wave `row` unpacks and stores line pair `row`
-    constexpr int np = 512 / 3;
-    const int ja = j0 + 2 * row, jb = ja + 1, my = a.rc.my, mgz = a.rc.mgalz;
-    const T2* Ar = A + row * RS;
-    const T hs = (T)(0.5 / 512.0);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const int ii = j + 64 * k;
-      if (ii < np) {
-        const T2 zk = Ar[ii];
-        T2 zc = Ar[(512 - ii) & 511];
-        zc.y = -zc.y;
-        T2 ya{(zk.x + zc.x) * hs, (zk.y + zc.y) * hs};
-        T2 yb{(zk.y - zc.y) * hs, -(zk.x - zc.x) * hs};  // (zk - zc) / (2i)
-        if (ii == 0) { ya.y = 0; yb.y = 0; }
-        const size_t base = ((size_t)ii * mgz + z) * a.rc.myp;
-        if (ja < my) dst[base + ja] = ya;
-        if (jb < my) dst[base + jb] = yb;
-      }
-    }
-  } else {
-    xl_unpack<T, T2, 512, 1>(a, A, dst, nullptr, z, j0, pairs);
-  }
-  xl_sync_x<T, T2>();
 }
 
 // Mean split: the transform inputs carry no 00 mode; its y-profile comes in
@@ -1049,14 +774,13 @@ __device__ __forceinline__ XlRk xl_rk(double dt, int rkstep) {
 // Compiled for two waves per SIMD (LOMA_XL_WPE; FP64 always): at three,
 // FP64 spills heavily (and its Z-transport build gave wrong results), and
 // FP32 spills enough to measure slower (3.33 vs 3.22 ms at 512x513x256).
-// XREG: the register-resident transform ends (FP32, 512 points, 4 pairs)
-template <typename T, bool WZ, int EPT, int NN, bool XREG>
+template <typename T, bool WZ, int EPT>
 __global__ __launch_bounds__(XL_THREADS)
 __attribute__((amdgpu_waves_per_eu(XL_THREADS == 512 ? 4 : (sizeof(T) == 8 ? 2 : LOMA_XL_WPE)))) void k_xline(FftArgs a) {
   const int bx = blockIdx.x;
 #include "loma_xline_body.inc"
 }
-template <typename T, bool WZ, int EPT, int NN, bool XREG>
+template <typename T, bool WZ, int EPT>
 __global__ __launch_bounds__(XL_THREADS)
 __attribute__((amdgpu_waves_per_eu(XL_THREADS == 512 ? 4 : (sizeof(T) == 8 ? 2 : LOMA_XL_WPE)))) void k_xline_batch(
     const FftArgs* __restrict__ args, const int* __restrict__ first, int nrun) {
@@ -1064,6 +788,296 @@ __attribute__((amdgpu_waves_per_eu(XL_THREADS == 512 ? 4 : (sizeof(T) == 8 ? 2 :
   const FftArgs& a = args[r];
   const int bx = blockIdx.x - first[r];
 #include "loma_xline_body.inc"
+}
+
+// ------------------------------------------------------------------------
+// x lines, a wavefront (or an aligned part of one) per transform row, for
+// rows of N = 64, 128, 256, 512 (E = 8) and 96, 192, 384 (E = 6) points.
+// RL = N / E lanes own a row, E entries each, jl + RL r: what the last inverse
+// pass (radix E) leaves in a lane's registers, what the physics takes there
+// and what the first forward pass (radix E) starts from.  The passes stay
+// inside the row's lanes and run in place in LDS between wavefront barriers;
+// workgroup barriers remain around the pack and the unpack, whose lanes walk
+// the y runs.  Rows carry one pad entry per eight and four more: pack, passes
+// and unpack of the powers of two are free of bank conflicts.  FP64 transforms
+// two fields at once (a thread holds 4 entries of each field, not 8: at 8 its
+// registers allow one wavefront per SIMD) and its waves exchange entries
+// through the rows.
+// Radices: E = 8: R0 = N / 64, 8, 8 (inverse), 8, 8, R0 (forward); E = 6:
+// 8, RB = N / 48, 6 and 6, 8, RB.
+// ------------------------------------------------------------------------
+__device__ __forceinline__ double uniform(double v) {
+  const long long b = __builtin_bit_cast(long long, v);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((int)b);
+  const unsigned hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+  return __builtin_bit_cast(double, (long long)(((unsigned long long)hi << 32) | lo));
+}
+template <typename T, int N_>
+struct XRow {
+  using T2 = typename std::conditional<sizeof(T) == 4, float2, double2>::type;
+  static constexpr int N = N_, NP = N / 3, E = N % 3 ? 8 : 6, RL = N / E;
+  static constexpr int R0 = N / 64, RB = N / 48;
+  static constexpr int NF = sizeof(T) == 8 ? 2 : 1;   // fields per transform
+  static constexpr int EF = E / NF;                   // entries of a thread per field
+  static constexpr int pairs_of(int cap) {            // line pairs: a power of two, at most 16
+    int p = 16;
+    while (p * N > cap) p /= 2;
+    return p;
+  }
+  static constexpr int P = pairs_of(sizeof(T) == 8 ? 1024 : 2048);
+  static constexpr int GT = P * RL, NT = NF * GT, ROWS = NF * P;
+  static constexpr int RS = N + N / 8 + 4;
+  static constexpr int NBUF = sizeof(T) == 8 ? 1 : 2;   // row buffers
+  static constexpr int XR = (NP * P + GT - 1) / GT;
+  static constexpr int NL = E == 8 ? (R0 > 1 ? 8 / R0 : 1) : (48 + RL - 1) / RL;
+  __device__ static __forceinline__ constexpr int li(int i) { return i + (i >> 3); }
+  // position of entry jl + RL r (RL is a multiple of 8)
+  __device__ static __forceinline__ int at(int jl, int r) { return li(jl) + RL / 8 * 9 * r; }
+  // first twiddles of the passes for lane jl
+  struct Tw {
+    T2 inv1, inv2, fwd1, fwd2[NL];
+  };
+  __device__ static __forceinline__ Tw twiddles(const T2* __restrict__ tw, int jl) {
+    Tw t;
+    t.inv1 = tw[E == 8 ? jl % R0 * (N / (8 * R0)) : jl % 8 * 6];
+    t.inv2 = tw[jl];
+    t.fwd1 = tw[jl % E * (N / (8 * E))];
+#pragma unroll
+    for (int q = 0; q < NL; ++q) t.fwd2[q] = tw[E == 8 || jl + RL * q < 48 ? jl + RL * q : 0];
+    return t;
+  }
+  // This thread's (kx, line pair) items of a field: byte offset in the field
+  // and the row entries X_k and X_{N-k} go to.  Items past the last read item
+  // 0 and write the pad entries behind the row, as X_N of kx = 0 does.
+  struct Items {
+    unsigned off[XR];
+    int lo[XR], hi[XR];
+  };
+  __device__ static __forceinline__ Items items(int tg, int mgz, int z, int myp, int j0, int my) {
+    Items t;
+#pragma unroll
+    for (int r = 0; r < XR; ++r) {
+      const int it = tg + r * GT;
+      const bool ok = it < NP * P;
+      const int ii = ok ? it / P : 0, q = it % P;
+      // tiles of up to 16 lines end inside the row's padding to a multiple of 16
+      const int j = 2 * P <= 16 || j0 + 2 * q < my ? j0 + 2 * q : j0;
+      t.off[r] = (((unsigned)ii * mgz + z) * myp + j) * (unsigned)sizeof(T2);
+      t.lo[r] = q * RS + (ok ? li(ii) : li(N) + 1);
+      t.hi[r] = q * RS + li(N - ii);
+    }
+    return t;
+  }
+  __device__ static __forceinline__ void fetch(const T2* __restrict__ src, const Items& t,
+                                               XlIn<T2, XR>& v) {
+    typedef T vec __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int r = 0; r < XR; ++r) {
+      const vec q = *(const vec*)((const char*)src + t.off[r]);
+      v.a[r] = T2{q[0], q[1]};
+      v.b[r] = T2{q[2], q[3]};
+    }
+  }
+  // two real lines to one complex row; the imaginary part of the kx = 0
+  // coefficient is ignored (rft, rftsingle.f:87-91).  left: lines of the tile
+  // inside the grid (the others read as zero)
+  __device__ static __forceinline__ void pack(XlIn<T2, XR> v, T2* A, int tg, const Items& t,
+                                              int left) {
+    if (left < 2 * P) {
+#pragma unroll
+      for (int r = 0; r < XR; ++r) {
+        const int l = 2 * ((tg + r * GT) % P);
+        v.a[r].x = l < left ? v.a[r].x : (T)0;
+        v.a[r].y = l < left ? v.a[r].y : (T)0;
+        v.b[r].x = l + 1 < left ? v.b[r].x : (T)0;
+        v.b[r].y = l + 1 < left ? v.b[r].y : (T)0;
+      }
+    }
+    v.a[0].y = tg < P ? (T)0 : v.a[0].y;
+    v.b[0].y = tg < P ? (T)0 : v.b[0].y;
+#pragma unroll
+    for (int r = 0; r < XR; ++r) {
+      const T2 ca = v.a[r], cb = v.b[r];
+      A[t.lo[r]] = T2{ca.x - cb.y, ca.y + cb.x};      // X_a + i X_b
+      A[t.hi[r]] = T2{ca.x + cb.y, -ca.y + cb.x};     // conj(X_a) + i conj(X_b)
+    }
+  }
+  // entry jl + c of a packed row (c a multiple of 8); NP .. N-NP are zero
+  // (dealiased) and not stored
+  __device__ static __forceinline__ T2 packed(const T2* A, int jl, int c) {
+    if (c >= NP && c + RL - 1 <= N - NP) return T2{0, 0};
+    const int i = jl + c;
+    if (c + RL <= NP || c > N - NP) return A[li(jl) + c / 8 * 9];
+    return i < NP || i > N - NP ? A[li(jl) + c / 8 * 9] : T2{0, 0};
+  }
+  __device__ static __forceinline__ void inverse(T2* A, int jl, const Tw& tw, T2 (&w)[E]) {
+    if constexpr (E == 8) {
+      if constexpr (R0 > 1) {
+#pragma unroll
+        for (int q = 0; q < 8 / R0; ++q)
+#pragma unroll
+          for (int r = 0; r < R0; ++r) w[q * R0 + r] = packed(A, jl, RL * q + 64 * r);
+        wave_sync();
+#pragma unroll
+        for (int q = 0; q < 8 / R0; ++q) {
+          dft_r<R0, T, T2>(w + q * R0, +1);
+          const int o = li((jl + RL * q) * R0);
+#pragma unroll
+          for (int r = 0; r < R0; ++r) A[o + r] = w[q * R0 + r];
+        }
+        wave_sync();
+      }
+#pragma unroll
+      for (int r = 0; r < 8; ++r) w[r] = R0 > 1 ? A[at(jl, r)] : packed(A, jl, RL * r);
+      if constexpr (R0 > 1) twiddle_pow<8>(w, tw.inv1, +1);
+      dft8<T, T2>(w, +1);
+      wave_sync();
+      const int o = li(jl / R0 * (R0 * 8) + jl % R0);
+#pragma unroll
+      for (int r = 0; r < 8; ++r) A[o + r * R0 + (r * R0 >> 3)] = w[r];
+    } else {
+      const bool on = jl < N / 8;
+      T2 u[8];
+      if (on) {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          const int i = jl + r * (N / 8);
+          u[r] = i < NP || i > N - NP ? A[li(i)] : T2{0, 0};
+        }
+      }
+      wave_sync();
+      if (on) {
+        dft8<T, T2>(u, +1);
+#pragma unroll
+        for (int r = 0; r < 8; ++r) A[9 * jl + r] = u[r];
+      }
+      wave_sync();
+      T2 v[NL * RB];
+#pragma unroll
+      for (int q = 0; q < NL; ++q)
+        if (48 % RL == 0 || jl + RL * q < 48)
+#pragma unroll
+          for (int r = 0; r < RB; ++r) v[q * RB + r] = A[li(jl) + RL / 8 * 9 * q + 54 * r];
+      wave_sync();
+#pragma unroll
+      for (int q = 0; q < NL; ++q)
+        if (48 % RL == 0 || jl + RL * q < 48) {
+          twiddle_pow<RB>(v + q * RB, tw.inv1, +1);
+          dft_r<RB, T, T2>(v + q * RB, +1);
+          const int j = jl + RL * q, o = j / 8 * (9 * RB) + j % 8;
+#pragma unroll
+          for (int r = 0; r < RB; ++r) A[o + 9 * r] = v[q * RB + r];
+        }
+    }
+    wave_sync();
+#pragma unroll
+    for (int r = 0; r < E; ++r) w[r] = A[at(jl, r)];
+    twiddle_pow<E>(w, tw.inv2, +1);
+    dft_r<E, T, T2>(w, +1);
+  }
+  __device__ static __forceinline__ void forward(T2* A, int jl, const Tw& tw, T2 (&w)[E]) {
+    dft_r<E, T, T2>(w, -1);
+#pragma unroll
+    for (int r = 0; r < E; ++r) A[E == 8 ? 9 * jl + r : li(6 * jl + r)] = w[r];
+    wave_sync();
+    if constexpr (E == 8) {
+#pragma unroll
+      for (int r = 0; r < 8; ++r) w[r] = A[at(jl, r)];
+      twiddle_pow<8>(w, tw.fwd1, -1);
+      dft8<T, T2>(w, -1);
+      wave_sync();
+      const int o = li(jl / 8 * 64 + jl % 8);
+#pragma unroll
+      for (int r = 0; r < 8; ++r) A[o + 9 * r] = w[r];
+      if constexpr (R0 > 1) {
+        wave_sync();
+#pragma unroll
+        for (int q = 0; q < NL; ++q)
+#pragma unroll
+          for (int r = 0; r < R0; ++r) w[q * R0 + r] = A[li(jl) + RL / 8 * 9 * q + 72 * r];
+#pragma unroll
+        for (int q = 0; q < NL; ++q) {
+          twiddle_pow<R0>(w + q * R0, tw.fwd2[q], -1);
+          dft_r<R0, T, T2>(w + q * R0, -1);
+        }
+        wave_sync();
+#pragma unroll
+        for (int q = 0; q < NL; ++q)
+#pragma unroll
+          for (int r = 0; r < R0; ++r) A[li(jl) + RL / 8 * 9 * q + 72 * r] = w[q * R0 + r];
+      }
+    } else {
+      const bool on = jl < N / 8;
+      T2 u[8];
+      if (on) {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) u[r] = A[li(jl + r * (N / 8))];
+      }
+      wave_sync();
+      if (on) {
+        twiddle_pow<8>(u, tw.fwd1, -1);
+        dft8<T, T2>(u, -1);
+        const int o = jl / 6 * 48 + jl % 6;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) A[li(o + 6 * r)] = u[r];
+      }
+      wave_sync();
+      // in place: an item's outputs are its inputs' entries
+#pragma unroll
+      for (int q = 0; q < NL; ++q)
+        if (48 % RL == 0 || jl + RL * q < 48) {
+          T2 v[RB];
+          const int o = li(jl) + RL / 8 * 9 * q;
+#pragma unroll
+          for (int r = 0; r < RB; ++r) v[r] = A[o + 54 * r];
+          twiddle_pow<RB>(v, tw.fwd2[q], -1);
+          dft_r<RB, T, T2>(v, -1);
+#pragma unroll
+          for (int r = 0; r < RB; ++r) A[o + 54 * r] = v[r];
+        }
+    }
+  }
+  // Hermitian unpacking into a field, scaled by 1/N (lines past my go to the
+  // row's padding, which is never read, or are dropped)
+  __device__ static __forceinline__ void unpack(const T2* A, T2* __restrict__ dst, int tg,
+                                                const Items& t, int left) {
+    typedef T vec __attribute__((ext_vector_type(4)));
+    const T hs = (T)(0.5 / (double)N);
+#pragma unroll
+    for (int r = 0; r < XR; ++r) {
+      const int it = tg + r * GT, q = it % P;
+      const T2 zk = A[t.lo[r]];
+      T2 zc = A[r == 0 && tg < P ? q * RS : t.hi[r]];
+      zc.y = -zc.y;
+      vec y;
+      y[0] = (zk.x + zc.x) * hs;
+      y[1] = (zk.y + zc.y) * hs;
+      y[2] = (zk.y - zc.y) * hs;  // (zk - zc) / (2i)
+      y[3] = -(zk.x - zc.x) * hs;
+      if (r == 0) {
+        y[1] = tg < P ? (T)0 : y[1];
+        y[3] = tg < P ? (T)0 : y[3];
+      }
+      if ((r < XR - 1 || it < NP * P) && (2 * P <= 16 || 2 * q < left))
+        *(vec*)((char*)dst + t.off[r]) = y;
+    }
+  }
+};
+
+template <typename T, bool WZ, int N>
+__global__ __launch_bounds__((XRow<T, N>::NT))
+__attribute__((amdgpu_waves_per_eu(2))) void k_xrow(FftArgs a) {
+  const int bx = blockIdx.x;
+#include "loma_xrow_body.inc"
+}
+template <typename T, bool WZ, int N>
+__global__ __launch_bounds__((XRow<T, N>::NT))
+__attribute__((amdgpu_waves_per_eu(2))) void k_xrow_batch(
+    const FftArgs* __restrict__ args, const int* __restrict__ first, int nrun) {
+  const int r = batch_run(first, nrun, blockIdx.x);
+  const FftArgs& a = args[r];
+  const int bx = blockIdx.x - first[r];
+#include "loma_xrow_body.inc"
 }
 
 // fourz on standalone rows (FFTPACK convention), for the per-operator API
@@ -1096,7 +1110,7 @@ static size_t zfft_lds(bool fp32, const FftArgs& a) {
 static size_t xline_lds(bool fp32, const FftArgs& a) {
   const int nf = fp32 ? xl_nf<float>() : xl_nf<double>();
   const int pad = fp32 ? xl_pad<float>() : xl_pad<double>();
-  return (size_t)2 * lds_entries(nf * (a.L / 2) * (a.rc.mgalx + LOMA_XL_RS1), pad) *
+  return (size_t)2 * lds_entries(nf * (a.L / 2) * a.rc.mgalx, pad) *
          (fp32 ? 8 : 16);
 }
 
@@ -1139,42 +1153,62 @@ int launch_zfft_fwd(bool fp32, const FftArgs& a, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
-// FP32 x lines at 512 points with 4 pairs take the register-resident
-// transform ends (LOMA_XL_REG32 = 0 turns them off)
-#ifndef LOMA_XL_REG32
-#define LOMA_XL_REG32 1
-#endif
-template <typename T, bool WZ, int E, int NN>
-static void launch_xline_nn(const FftArgs& a, dim3 g, dim3 b, size_t lds, hipStream_t st) {
-  if constexpr (sizeof(T) == 4 && NN == 512 && E == 8 && LOMA_XL_REG32 && xl_pad<T>() == 0 &&
-                xl_nf<T>() == 1) {
-    if (a.L == 8) {
-      hipLaunchKernelGGL((k_xline<T, WZ, E, NN, true>), g, b, lds, st, a);
-      return;
-    }
+// k_xrow serves the production lengths at the tile the plan gives them
+// (L = 2 P lines) and fields under 4 GiB (32-bit offsets in a field); other
+// lengths, tiles and sizes take k_xline with its run-time plan.
+template <typename T>
+static bool xrow_tile(const FftArgs& a) {
+  switch (a.rc.mgalx) {
+    case 64: return a.L == 2 * XRow<T, 64>::P;
+    case 96: return a.L == 2 * XRow<T, 96>::P;
+    case 128: return a.L == 2 * XRow<T, 128>::P;
+    case 192: return a.L == 2 * XRow<T, 192>::P;
+    case 256: return a.L == 2 * XRow<T, 256>::P;
+    case 384: return a.L == 2 * XRow<T, 384>::P;
+    case 512: return a.L == 2 * XRow<T, 512>::P;
+    default: return false;
   }
-  hipLaunchKernelGGL((k_xline<T, WZ, E, NN, false>), g, b, lds, st, a);
+}
+bool xrow_serves(bool fp32, const FftArgs& a) {
+  const unsigned long long field = (unsigned long long)a.rc.nplanes * a.rc.mgalz * a.rc.myp;
+  return field * (fp32 ? 8 : 16) < (1ull << 32) &&
+         (fp32 ? xrow_tile<float>(a) : xrow_tile<double>(a));
+}
+
+// x-line kernel of a run's length
+#define LOMA_XROW_BY_LENGTH(n, LAUNCH)                   \
+  switch (n) {                                           \
+    case 64: { constexpr int NN = 64; LAUNCH; break; }   \
+    case 96: { constexpr int NN = 96; LAUNCH; break; }   \
+    case 128: { constexpr int NN = 128; LAUNCH; break; } \
+    case 192: { constexpr int NN = 192; LAUNCH; break; } \
+    case 256: { constexpr int NN = 256; LAUNCH; break; } \
+    case 384: { constexpr int NN = 384; LAUNCH; break; } \
+    case 512: { constexpr int NN = 512; LAUNCH; break; } \
+  }
+
+template <typename T, bool WZ>
+static void launch_xline_t(const FftArgs& a, dim3 g, size_t lds, hipStream_t st) {
+  // entries per thread of k_xline: pairs * mgalx <= XL_THREADS * EPT, i.e. at
+  // most 1024 (FP64) / 2048 (FP32) entries per workgroup (checked at init)
+  constexpr int EPT = (sizeof(T) == 8 ? 1024 : 2048) / XL_THREADS;
+  if (a.xrow) {
+    LOMA_XROW_BY_LENGTH(a.rc.mgalx, hipLaunchKernelGGL((k_xrow<T, WZ, NN>), g, dim3(XRow<T, NN>::NT), 0, st, a));
+  } else {
+    hipLaunchKernelGGL((k_xline<T, WZ, EPT>), g, dim3(XL_THREADS), lds, st, a);
+  }
 }
 
 int launch_xline(bool fp32, const FftArgs& a, hipStream_t st) {
   const int nyb = (a.rc.my + a.L - 1) / a.L;
-  dim3 g(xcd_groups(a.rc.mgalz * nyb)), b(XL_THREADS);
+  dim3 g(xcd_groups(a.rc.mgalz * nyb));
   const size_t lds = xline_lds(fp32, a);
-  // entries per thread: pairs * mgalx <= XL_THREADS * EPT, i.e. at most
-  // 1024 (FP64) / 2048 (FP32) entries per workgroup (checked at init)
-  constexpr int E64 = 1024 / XL_THREADS, E32 = 2048 / XL_THREADS;
   if (fp32) {
-    if (a.with_z) {
-      LOMA_BY_LENGTH(a.rc.mgalx, (launch_xline_nn<float, true, E32, NN>(a, g, b, lds, st)));
-    } else {
-      LOMA_BY_LENGTH(a.rc.mgalx, (launch_xline_nn<float, false, E32, NN>(a, g, b, lds, st)));
-    }
+    if (a.with_z) launch_xline_t<float, true>(a, g, lds, st);
+    else launch_xline_t<float, false>(a, g, lds, st);
   } else {
-    if (a.with_z) {
-      LOMA_BY_LENGTH(a.rc.mgalx, (launch_xline_nn<double, true, E64, NN>(a, g, b, lds, st)));
-    } else {
-      LOMA_BY_LENGTH(a.rc.mgalx, (launch_xline_nn<double, false, E64, NN>(a, g, b, lds, st)));
-    }
+    if (a.with_z) launch_xline_t<double, true>(a, g, lds, st);
+    else launch_xline_t<double, false>(a, g, lds, st);
   }
   return (int)hipGetLastError();
 }
@@ -1206,38 +1240,28 @@ int launch_zfft_batch(bool fp32, bool inv, const FftArgs& proto, const FftArgs* 
   return (int)hipGetLastError();
 }
 
-template <typename T, bool WZ, int E, int NN>
-static void launch_xline_batch_nn(const FftArgs& proto, dim3 g, dim3 b, size_t lds,
-                                  hipStream_t st, const FftArgs* args, const int* first,
-                                  int nrun) {
-  if constexpr (sizeof(T) == 4 && NN == 512 && E == 8 && LOMA_XL_REG32 && xl_pad<T>() == 0 &&
-                xl_nf<T>() == 1) {
-    if (proto.L == 8) {
-      hipLaunchKernelGGL((k_xline_batch<T, WZ, E, NN, true>), g, b, lds, st, args, first, nrun);
-      return;
-    }
+template <typename T, bool WZ>
+static void launch_xline_batch_t(const FftArgs& proto, dim3 g, size_t lds, hipStream_t st,
+                                 const FftArgs* args, const int* first, int nrun) {
+  constexpr int EPT = (sizeof(T) == 8 ? 1024 : 2048) / XL_THREADS;
+  if (proto.xrow) {
+    LOMA_XROW_BY_LENGTH(proto.rc.mgalx, hipLaunchKernelGGL((k_xrow_batch<T, WZ, NN>), g, dim3(XRow<T, NN>::NT), 0, st, args, first, nrun));
+  } else {
+    hipLaunchKernelGGL((k_xline_batch<T, WZ, EPT>), g, dim3(XL_THREADS), lds, st, args, first, nrun);
   }
-  hipLaunchKernelGGL((k_xline_batch<T, WZ, E, NN, false>), g, b, lds, st, args, first, nrun);
 }
 
 int launch_xline_batch(bool fp32, const FftArgs& proto, const FftArgs* args, const int* first,
                        int nrun, int nblocks, hipStream_t st) {
   if (nblocks <= 0 || nrun <= 0) return 0;
-  dim3 g(nblocks), b(XL_THREADS);
+  dim3 g(nblocks);
   const size_t lds = xline_lds(fp32, proto);
-  constexpr int E64 = 1024 / XL_THREADS, E32 = 2048 / XL_THREADS;
   if (fp32) {
-    if (proto.with_z) {
-      LOMA_BY_LENGTH(proto.rc.mgalx, (launch_xline_batch_nn<float, true, E32, NN>(proto, g, b, lds, st, args, first, nrun)));
-    } else {
-      LOMA_BY_LENGTH(proto.rc.mgalx, (launch_xline_batch_nn<float, false, E32, NN>(proto, g, b, lds, st, args, first, nrun)));
-    }
+    if (proto.with_z) launch_xline_batch_t<float, true>(proto, g, lds, st, args, first, nrun);
+    else launch_xline_batch_t<float, false>(proto, g, lds, st, args, first, nrun);
   } else {
-    if (proto.with_z) {
-      LOMA_BY_LENGTH(proto.rc.mgalx, (launch_xline_batch_nn<double, true, E64, NN>(proto, g, b, lds, st, args, first, nrun)));
-    } else {
-      LOMA_BY_LENGTH(proto.rc.mgalx, (launch_xline_batch_nn<double, false, E64, NN>(proto, g, b, lds, st, args, first, nrun)));
-    }
+    if (proto.with_z) launch_xline_batch_t<double, true>(proto, g, lds, st, args, first, nrun);
+    else launch_xline_batch_t<double, false>(proto, g, lds, st, args, first, nrun);
   }
   return (int)hipGetLastError();
 }

@@ -118,6 +118,7 @@ struct FftArgs {
   int with_z;
   int J;                     // y rows per z-transform block
   int L;                     // lines per x-line block
+  int xrow;                  // x lines by k_xrow (xrow_serves)
 };
 
 // statistics window (addstats1/2 and the phys2 sums of cross.f): the
@@ -218,6 +219,9 @@ int zfft_blocks(const FftArgs& a);
 int xline_blocks(const FftArgs& a);
 
 int launch_zfft_inv(bool fp32, const FftArgs& a, hipStream_t st);
+// whether the run's length, tile and size take the row kernel (the caller
+// sets a.xrow)
+bool xrow_serves(bool fp32, const FftArgs& a);
 int launch_xline(bool fp32, const FftArgs& a, hipStream_t st);
 int launch_zfft_fwd(bool fp32, const FftArgs& a, hipStream_t st);
 int launch_fourz(const FftPlan& pl, const double2* tw, double2* c, int nrows, int iopt,
