@@ -115,6 +115,11 @@ struct loma_run {
   double *st_acc = nullptr, *st_spe = nullptr, *st_part = nullptr, *st_rho = nullptr,
          *st_last = nullptr;
   int* st_jsp = nullptr;
+  // workspace of the batched solves (solve_ws)
+  std::mutex ws_mu;
+  void* ws = nullptr;
+  size_t ws_bytes = 0;
+  hipEvent_t ws_ev = nullptr;
   int st_nsp = 0;
   bool st_on = false;
   int st_nacum = 0;
@@ -318,6 +323,8 @@ int loma_free(loma_run* r) {
   pinned_put(r->hstage, r->hstage_n * sizeof(double));
   if (r->arena) hipFree(r->arena);
   if (r->snap) hipFree(r->snap);
+  if (r->ws) hipFree(r->ws);
+  if (r->ws_ev) hipEventDestroy(r->ws_ev);
   for (void* p : {(void*)r->st_acc, (void*)r->st_spe, (void*)r->st_part, (void*)r->st_rho,
                   (void*)r->st_last, (void*)r->st_jsp})
     if (p) hipFree(p);
@@ -426,21 +433,22 @@ int loma_init(loma_run** out, int mgalx, int my, int mgalz, const double* y, dou
     h[o + stream_index(n, e, l, 2)] = v;
     h32[o + stream_index(n, e, l, 4)] = (float)v;
   };
-  auto put_at = [&](int id, int row, int idx, double v) {
-    const int w = ytab_width(id), l = row / M, t = row - l * M;
-    set(ytab_offset(id, M), w * M, t * w + idx, l, v);
-  };
   // row-indexed source -> table entries i0 .. i0+w-1 of each row
   auto put = [&](int id, const std::vector<double>& src, int w, int i0) {
-    for (int j = 0; j < my; ++j)
-      for (int d = 0; d < w; ++d) put_at(id, j, i0 + d, src[(size_t)j * w + d]);
+    const int W = ytab_width(id), o = ytab_offset(id, M);
+    for (int j = 0, l = 0, t = 0; j < my; ++j) {
+      for (int d = 0; d < w; ++d) set(o, W * M, t * W + i0 + d, l, src[(size_t)j * w + d]);
+      if (++t == M) { t = 0; ++l; }
+    }
   };
   // lower multipliers: lo[k][i-1] (row k into row k+i) -> destination row k+i
   auto put_lo = [&](int id, const std::vector<double>& src) {
-    const int w = ytab_width(id);
-    for (int j = 0; j < my; ++j)
-      for (int i = 1; i <= w; ++i)
-        if (j - i >= 0) put_at(id, j, i - 1, src[(size_t)(j - i) * w + i - 1]);
+    const int W = ytab_width(id), o = ytab_offset(id, M);
+    for (int j = 0, l = 0, t = 0; j < my; ++j) {
+      for (int i = 1; i <= W && j - i >= 0; ++i)
+        set(o, W * M, t * W + i - 1, l, src[(size_t)(j - i) * W + i - 1]);
+      if (++t == M) { t = 0; ++l; }
+    }
   };
   put(YT_B1, f.b1, 7, 0); put(YT_A1, f.a1, 7, 0); put(YT_U1, f.inv1, 1, 0);
   put(YT_U1, f.up1, 3, 1); put_lo(YT_LO1, f.lo1); put(YT_FMAP, f.fmap, 1, 0);
@@ -450,13 +458,12 @@ int loma_init(loma_run** out, int mgalx, int my, int mgalz, const double* y, dou
   // scan compositions, [level][P*P][lane] -> one stream a level
   std::vector<double> hs((size_t)6 * 9 * 64);
   auto scan = [&](int id, bool upper, const double* lo, const double* up, const double* inv) {
-    const int P = ytab_width(id);
+    const int P = ytab_width(id), o = ytab_offset(id, M);
     const int lev = scan_table(my, M, P, upper, lo, up, inv, hs.data());
-    for (int k = 0; k < 6; ++k)
+    for (int k = 0; k < lev; ++k)
       for (int e = 0; e < P * P; ++e)
         for (int l = 0; l < 64; ++l)
-          set(ytab_offset(id, M) + (size_t)k * P * P * 64, P * P, e, l,
-              hs[((size_t)k * P * P + e) * 64 + l]);
+          set(o + k * P * P * 64, P * P, e, l, hs[((size_t)k * P * P + e) * 64 + l]);
     return lev;
   };
   int lev[6];
@@ -512,7 +519,7 @@ int loma_init(loma_run** out, int mgalx, int my, int mgalz, const double* y, dou
     if ((rc = dalloc(r, &r->helm_h, sizeof(double) * 2 * R * (size_t)r->nclass))) {
       loma_free(r); return rc;
     }
-    if (launch_helm_factor(r->dt21, r->dt22, my, M, dsh, r->nclass, r->helm_lu, sst) ||
+    if (launch_helm_factor(r->dt21, r->dt22, my, M, dsh, 0.0, r->nclass, r->helm_lu, sst) ||
         launch_helm_bc(M, r->T, r->helm_lu, r->helm_bc, r->helm_h, r->nclass, sst) ||
         hipStreamSynchronize(sst) != hipSuccess) {
       set_error("loma_init: factor launch failed"); loma_free(r); return LOMA_ERR_DEVICE;
@@ -1870,30 +1877,67 @@ int loma_deryyr2_dev(loma_run* r, const double* u, double* du, int ncols) {
   return LOMA_OK;
 }
 
+// Device workspace of the batched solves: the LU tables of `ncols` columns, at
+// most SOLVE_WS_MAX bytes (larger batches go through it in pieces), kept with
+// the run, grown on demand and freed with it.  One call at a time uses it
+// (ws_mu); the calls wait for their work before they return.
+constexpr size_t SOLVE_WS_MAX = (size_t)256 << 20;
+static int solve_ws(loma_run* r, int ncols, int per_col, int* chunk) {
+  const size_t one = sizeof(double) * (size_t)r->lu_stride * per_col;
+  const size_t fit = std::max<size_t>(1, SOLVE_WS_MAX / one);
+  *chunk = (int)std::min<size_t>((size_t)ncols, fit);
+  const size_t need = one * (size_t)*chunk;
+  if (r->ws_bytes < need) {
+    std::lock_guard<std::recursive_mutex> lk(g_setup_mu);
+    if (r->ws) {
+      HIPCHK(hipStreamSynchronize(r->stream));
+      HIPCHK(hipFree(r->ws));
+      r->ws = nullptr;
+      r->ws_bytes = 0;
+    }
+    if (hipMalloc(&r->ws, need) != hipSuccess) {
+      r->ws = nullptr;
+      set_error("solve workspace: device allocation failed");
+      return LOMA_ERR_OOM;
+    }
+    r->ws_bytes = need;
+  }
+  return LOMA_OK;
+}
+// The run's stream waits for work already on the null stream (the caller's
+// inputs may be on their way there).
+static int after_null_stream(loma_run* r) {
+  std::lock_guard<std::recursive_mutex> lk(g_setup_mu);
+  if (!r->ws_ev) HIPCHK(hipEventCreateWithFlags(&r->ws_ev, hipEventDisableTiming));
+  HIPCHK(hipEventRecord(r->ws_ev, nullptr));
+  HIPCHK(hipStreamWaitEvent(r->stream, r->ws_ev, 0));
+  return LOMA_OK;
+}
+
 static int solve_cols(loma_run* r, const double* phi, double* v, double* dvdy,
                       const double* rK, double shift, int ncols, int mode) {
   if (!r || ncols < 0) return LOMA_ERR_ARG;
   if (ncols == 0) return LOMA_OK;
-  std::vector<double> h(ncols);
-  HIPCHK(hipMemcpy(h.data(), rK, sizeof(double) * ncols, hipMemcpyDeviceToHost));
-  for (double& x : h) x += shift;
-  double *sh = nullptr, *lu = nullptr, *bc = nullptr;
-  HIPCHK(hipMalloc(&sh, sizeof(double) * ncols));
-  HIPCHK(hipMalloc(&lu, sizeof(double) * (size_t)r->lu_stride * ncols));
-  HIPCHK(hipMalloc(&bc, sizeof(double) * 4 * (size_t)ncols));
-  int rc = LOMA_OK;
-  if (hipMemcpy(sh, h.data(), sizeof(double) * ncols, hipMemcpyHostToDevice) != hipSuccess ||
-      launch_helm_factor(r->dt21, r->dt22, r->my, r->M, sh, ncols, lu, r->stream) ||
-      launch_helm_bc(r->M, r->T, lu, bc, nullptr, ncols, r->stream) ||
-      launch_lapvdvhom(r->M, r->T, lu, bc, phi, v, dvdy, rK, ncols, mode, r->stream) ||
-      hipStreamSynchronize(r->stream) != hipSuccess) {
-    set_error("solve_cols: device failure");
-    rc = LOMA_ERR_DEVICE;
+  std::lock_guard<std::mutex> lk(r->ws_mu);
+  int chunk = 0;
+  int e = solve_ws(r, ncols, 1, &chunk);
+  if (!e) e = after_null_stream(r);
+  if (e) return e;
+  double* lu = (double*)r->ws;
+  int rc = 0;
+  for (int c = 0; c < ncols && !rc; c += chunk) {
+    const int n = std::min(chunk, ncols - c);
+    const size_t o = 2 * (size_t)c * r->my;
+    rc = launch_helm_factor(r->dt21, r->dt22, r->my, r->M, rK + c, shift, n, lu, r->stream);
+    if (!rc)
+      rc = launch_lapvdvhom(r->M, r->T, lu, phi + o, v + o, dvdy ? dvdy + o : nullptr, rK + c, n,
+                            mode, r->stream);
   }
-  hipFree(sh);
-  hipFree(lu);
-  hipFree(bc);
-  return rc;
+  if (rc || hipStreamSynchronize(r->stream) != hipSuccess) {
+    set_error("solve_cols: device failure");
+    return LOMA_ERR_DEVICE;
+  }
+  return LOMA_OK;
 }
 
 int loma_lapvdvhom_dev(loma_run* r, const double* phi, double* v, double* dvdy,
@@ -1914,27 +1958,28 @@ int loma_visc_dev(loma_run* r, double* vorwk, double* vor, double* phi, double* 
   if (!r || ncols < 0 || !vorwk || !vor || !phi || !v || !dvdy || !phiwk || !rk1 || !rk2)
     return LOMA_ERR_ARG;
   if (ncols == 0) return LOMA_OK;
-  double *lu = nullptr, *bc = nullptr;
-  const size_t L = (size_t)r->lu_stride * ncols;
-  HIPCHK(hipMalloc(&lu, sizeof(double) * 2 * L));
-  if (hipMalloc(&bc, sizeof(double) * 4 * (size_t)ncols) != hipSuccess) {
-    hipFree(lu);
-    set_error("loma_visc_dev: allocation failed");
-    return LOMA_ERR_OOM;
+  std::lock_guard<std::mutex> lk(r->ws_mu);
+  int chunk = 0;
+  int e = solve_ws(r, ncols, 2, &chunk);
+  if (!e) e = after_null_stream(r);
+  if (e) return e;
+  int rc = 0;
+  for (int c = 0; c < ncols && !rc; c += chunk) {
+    const int n = std::min(chunk, ncols - c);
+    const size_t o = 2 * (size_t)c * r->my;
+    double* lu1 = (double*)r->ws;
+    double* lu2 = lu1 + (size_t)r->lu_stride * n;
+    rc = launch_helm_factor(r->dt21, r->dt22, r->my, r->M, rk1 + c, 0.0, n, lu1, r->stream);
+    if (!rc) rc = launch_helm_factor(r->dt21, r->dt22, r->my, r->M, rk2 + c, 0.0, n, lu2, r->stream);
+    if (!rc)
+      rc = launch_visc(r->M, r->T, lu1, lu2, vorwk + o, vor + o, phi + o, v + o, dvdy + o,
+                       phiwk + o, rk2 + c, dalbe, dtri, dtxi, n, r->stream);
   }
-  int rc = LOMA_OK;
-  if (launch_helm_factor(r->dt21, r->dt22, r->my, r->M, rk1, ncols, lu, r->stream) ||
-      launch_helm_factor(r->dt21, r->dt22, r->my, r->M, rk2, ncols, lu + L, r->stream) ||
-      launch_helm_bc(r->M, r->T, lu + L, bc, nullptr, ncols, r->stream) ||
-      launch_visc(r->M, r->T, lu, lu + L, bc, vorwk, vor, phi, v, dvdy, phiwk, rk2, dalbe,
-                  dtri, dtxi, ncols, r->stream) ||
-      hipStreamSynchronize(r->stream) != hipSuccess) {
+  if (rc || hipStreamSynchronize(r->stream) != hipSuccess) {
     set_error("loma_visc_dev: device failure");
-    rc = LOMA_ERR_DEVICE;
+    return LOMA_ERR_DEVICE;
   }
-  hipFree(lu);
-  hipFree(bc);
-  return rc;
+  return LOMA_OK;
 }
 
 int loma_inty8_dev(loma_run* r, const double* du, double* u) {

@@ -151,18 +151,18 @@ struct StatsArgs {
 int launch_dy(int M, int order, const YTab& T, const double* u, double* du, int ncols,
               hipStream_t st);
 int launch_helm_factor(const double* dt21, const double* dt22, int my, int M,
-                       const double* shifts, int nsys, double* lu, hipStream_t st);
+                       const double* shifts, double shift, int nsys, double* lu,
+                       hipStream_t st);
 // per-class Neumann constants (bc, 4 per class) and, when h is not null,
 // the homogeneous solutions h1 = LU^-1 e_0, h2 = LU^-1 e_{my-1} of each
 // class (lane-major, 2 entries per row, 2*64*M doubles per class)
 int launch_helm_bc(int M, const YTab& T, const double* lu, double* bc, double* h, int nclass,
                    hipStream_t st);
-int launch_lapvdvhom(int M, const YTab& T, const double* lu, const double* bc,
-                     const double* phi, double* v, double* dv, const double* rK,
-                     int ncols, int mode, hipStream_t st);
+int launch_lapvdvhom(int M, const YTab& T, const double* lu, const double* phi, double* v,
+                     double* dv, const double* rK, int ncols, int mode, hipStream_t st);
 int launch_inty8(int M, const YTab& T, const double* du, double* u, hipStream_t st);
-int launch_visc(int M, const YTab& T, const double* lu1, const double* lu2, const double* bc2,
-                double* vorwk, double* vor, double* phi, double* v, double* dvdy,
+int launch_visc(int M, const YTab& T, const double* lu1, const double* lu2, double* vorwk,
+                double* vor, double* phi, double* v, double* dvdy,
                 double* phiwk, const double* rk2, double dalbe, double dtri, double dtxi,
                 int ncols, hipStream_t st);
 

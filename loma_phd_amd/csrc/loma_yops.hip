@@ -10,16 +10,16 @@ namespace loma {
 template <int M>
 int launch_dy_m(int, const YTab&, const double*, double*, int, hipStream_t);
 template <int M>
-int launch_lapvdvhom_m(const YTab&, const double*, int, const double*, const double*,
-                       double*, double*, const double*, int, int, hipStream_t);
+int launch_lapvdvhom_m(const YTab&, const double*, int, const double*, double*, double*,
+                       const double*, int, int, hipStream_t);
 template <int M>
 int launch_helm_bc_m(const YTab&, const double*, int, double*, double*, int, hipStream_t);
 template <int M>
 int launch_inty8_m(const YTab&, const double*, double*, hipStream_t);
 template <int M>
-int launch_visc_m(const YTab&, const double*, const double*, int, const double*, double*,
-                  double*, double*, double*, double*, double*, const double*, double, double,
-                  double, int, hipStream_t);
+int launch_visc_m(const YTab&, const double*, const double*, int, double*, double*, double*,
+                  double*, double*, double*, const double*, double, double, double, int,
+                  hipStream_t);
 template <int M>
 int launch_phase_m(int, bool, const PhaseArgs&, hipStream_t);
 template <int M>
@@ -67,12 +67,11 @@ int launch_dy(int M, int order, const YTab& T, const double* u, double* du, int 
   if (ncols <= 0) return 0;
   LOMA_DISPATCH_M(M, launch_dy_m<MM>(order, T, u, du, ncols, st));
 }
-int launch_lapvdvhom(int M, const YTab& T, const double* lu, const double* bc,
-                     const double* phi, double* v, double* dv, const double* rK, int ncols,
-                     int mode, hipStream_t st) {
+int launch_lapvdvhom(int M, const YTab& T, const double* lu, const double* phi, double* v,
+                     double* dv, const double* rK, int ncols, int mode, hipStream_t st) {
   if (ncols <= 0) return 0;
-  LOMA_DISPATCH_M(M, launch_lapvdvhom_m<MM>(T, lu, 5 * WAVE * MM, bc, phi, v, dv, rK, ncols,
-                                            mode, st));
+  LOMA_DISPATCH_M(M, launch_lapvdvhom_m<MM>(T, lu, 5 * WAVE * MM, phi, v, dv, rK, ncols, mode,
+                                            st));
 }
 int launch_helm_bc(int M, const YTab& T, const double* lu, double* bc, double* h, int nclass,
                    hipStream_t st) {
@@ -82,12 +81,12 @@ int launch_helm_bc(int M, const YTab& T, const double* lu, double* bc, double* h
 int launch_inty8(int M, const YTab& T, const double* du, double* u, hipStream_t st) {
   LOMA_DISPATCH_M(M, launch_inty8_m<MM>(T, du, u, st));
 }
-int launch_visc(int M, const YTab& T, const double* lu1, const double* lu2, const double* bc2,
-                double* vorwk, double* vor, double* phi, double* v, double* dvdy,
+int launch_visc(int M, const YTab& T, const double* lu1, const double* lu2, double* vorwk,
+                double* vor, double* phi, double* v, double* dvdy,
                 double* phiwk, const double* rk2, double dalbe, double dtri, double dtxi,
                 int ncols, hipStream_t st) {
   if (ncols <= 0) return 0;
-  LOMA_DISPATCH_M(M, launch_visc_m<MM>(T, lu1, lu2, 5 * WAVE * MM, bc2, vorwk, vor, phi, v,
+  LOMA_DISPATCH_M(M, launch_visc_m<MM>(T, lu1, lu2, 5 * WAVE * MM, vorwk, vor, phi, v,
                                        dvdy, phiwk, rk2, dalbe, dtri, dtxi, ncols, st));
 }
 int launch_phaseA(int M, bool fp32, const PhaseArgs& a, hipStream_t st) {
@@ -121,59 +120,150 @@ int launch_thickness(int M, bool fp32, const PhaseArgs& a, const double* hy, dou
   LOMA_DISPATCH_M(M, launch_thickness_m<MM>(fp32, a, hy, ly, which, st));
 }
 
-// LU of (dt22 - s dt21) with identity end rows (Lapvdvhom laps.f:349-366),
-// one thread per shift s.  Output per class: lane-major streams over 64*M
-// rows, first lo1, lo2 (lower multipliers by destination row), then inv, up1,
-// up2; zero beyond row my-1.
-__global__ void k_helm_factor(const double* __restrict__ dt21,
-                              const double* __restrict__ dt22, int my, int M,
-                              const double* __restrict__ shifts, int nsys,
-                              double* __restrict__ lu) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= nsys) return;
-  const double sh = shifts[s];
-  const int stride = 5 * WAVE * M;
-  double* out = lu + (size_t)s * stride;
-  for (int q = 0; q < stride; ++q) out[q] = 0.0;
-  // idx: 0 inv, 1 up1, 2 up2, 3 lo1, 4 lo2
-  auto at = [&](int row, int idx) -> double& {
-    const int l = row / M, t = row - l * M;
-    return idx < 3 ? out[2 * WAVE * M + stream_index(3 * M, t * 3 + idx, l, 2)]
-                   : out[stream_index(2 * M, t * 2 + idx - 3, l, 2)];
-  };
-  auto row = [&](int j, double* r) {
-    if (j >= my) { for (int d = 0; d < 5; ++d) r[d] = 0.0; return; }
-    if (j == 0 || j == my - 1) {
-      for (int d = 0; d < 5; ++d) r[d] = 0.0;
-      r[2] = 1.0;
-      return;
+// LU of (dt22 - s dt21), s = shifts[.] + shift, with identity end rows
+// (Lapvdvhom laps.f:349-366), one thread per system.  Output per system:
+// lane-major streams over 64*M rows, first lo1, lo2 (lower multipliers by
+// destination row), then inv, up1, up2; zero beyond row my-1.
+// The rows are a serial chain, and with a few wavefronts on the card its
+// instructions are what it costs: the band rows wait in LDS and are read one
+// row ahead, the three rows in flight rotate by name (no moves), the interior
+// rows run without edge tests, and stores take a scalar offset.
+// 92 -> 36 us for 441 systems of 129 rows and 230 -> 67 us for 7,225 of 257,
+// against one that cleared its tables first and walked them with index
+// divisions (64 or fewer systems a wavefront make no difference).
+__global__ __launch_bounds__(64) void k_helm_factor(const double* __restrict__ dt21,
+                                                    const double* __restrict__ dt22, int my,
+                                                    int M, const double* __restrict__ shifts,
+                                                    double shift, int nsys,
+                                                    double* __restrict__ lu) {
+  extern __shared__ __align__(16) double g[];  // rows of dt22, then of dt21
+  for (int q0 = threadIdx.x; q0 < 5 * my; q0 += 64 * 8) {
+    double c2[8], c1[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int q = min(q0 + 64 * i, 5 * my - 1);
+      c2[i] = dt22[q];
+      c1[i] = dt21[q];
     }
-    for (int d = 0; d < 5; ++d) r[d] = dt22[j * 5 + d] - sh * dt21[j * 5 + d];
-  };
-  double w[3][5];
-  row(0, w[0]); row(1, w[1]); row(2, w[2]);
-  for (int k = 0; k < my; ++k) {
-    const double iv = 1.0 / w[0][2];
-    at(k, 0) = iv;
-    at(k, 1) = (k + 1 < my) ? w[0][3] : 0.0;
-    at(k, 2) = (k + 2 < my) ? w[0][4] : 0.0;
-    for (int i = 1; i <= 2; ++i) {
-      if (k + i >= my) continue;
-      const double l = w[i][2 - i] * iv;
-      at(k + i, 2 + i) = l;  // multiplier of row k into row k+i
-      w[i][2 - i] = 0.0;
-      for (int d = 1; d <= 2; ++d) w[i][2 - i + d] -= l * w[0][2 + d];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int q = min(q0 + 64 * i, 5 * my - 1);
+      g[q] = c2[i];
+      g[5 * my + q] = c1[i];
     }
-    for (int d = 0; d < 5; ++d) { w[0][d] = w[1][d]; w[1][d] = w[2][d]; }
-    row(k + 3, w[2]);
   }
+  __syncthreads();
+  const int s = blockIdx.x * 64 + threadIdx.x;
+  if (s >= nsys) return;
+  const double sh = shifts[s] + shift;
+  const int stride = 5 * WAVE * M * 8;  // bytes of a system's table
+  const auto out = make_rsrc(lu + (size_t)blockIdx.x * 64 * (5 * WAVE * M), 0x7fffffff);
+  const int vo = threadIdx.x * stride;
+  auto put = [&](int so, double v) {
+    typedef unsigned u2v __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2v, v), out, vo, so, 0);
+  };
+  auto put_lo = [&](int l, int t, double a, double b) {
+    typedef unsigned u4v __attribute__((ext_vector_type(4)));
+    typedef double d2v __attribute__((ext_vector_type(2)));
+    d2v v;
+    v[0] = a;
+    v[1] = b;
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4v, v), out, vo,
+                                           (t * WAVE + l) * 16, 0);
+  };
+  int l = 0, t = 0, ln = 0, tn = 1;  // lane and slot of rows k and k+1 (M >= 3)
+  double l2 = 0.0;                   // row k-1's multiplier into row k+1
+  const int ubase = 2 * WAVE * M * 8, utail = ubase + (3 * M - 1) * (WAVE * 8);
+  const int tlast = (M & 1) ? M - 1 : -1;  // slot whose up2 lies behind the vectors
+  auto store_row = [&](double iv, double u1, double u2, double m1, double m2) {
+    // entries 3t .. 3t+2 of lane l's U stream, two to a 16-byte vector
+    const int odd = t & 1, ub = ubase + ((3 * t) >> 1) * (WAVE * 16) + l * 16;
+    const int in = ub + WAVE * 16 + odd * 8, tail = utail + l * 8;
+    put(ub + odd * 8, iv);
+    put(ub + 8 + odd * (WAVE * 16 - 8), u1);
+    put(t == tlast ? tail : in, u2);
+    if (ln < WAVE) put_lo(ln, tn, m1, l2);
+    l2 = m2;
+    const bool wrap = tn + 1 == M;
+    l = ln;
+    t = tn;
+    tn = wrap ? 0 : tn + 1;
+    ln = wrap ? ln + 1 : ln;
+  };
+  double n2[5], n1[5];               // the row after those in flight
+  auto ahead = [&](int j) {
+    const double* p = g + 5 * j;
+#pragma unroll
+    for (int d = 0; d < 5; ++d) {
+      n2[d] = p[d];
+      n1[d] = p[5 * my + d];
+    }
+  };
+  auto interior = [&](double (&r)[5]) {
+#pragma unroll
+    for (int d = 0; d < 5; ++d) r[d] = n2[d] - sh * n1[d];
+  };
+  // eliminates column k (pivot row a) from rows b and c
+  auto eliminate = [&](const double (&a)[5], double (&b)[5], double (&c)[5], double& iv,
+                       double& m1, double& m2) {
+    iv = 1.0 / a[2];
+    m1 = b[1] * iv;
+    b[2] -= m1 * a[3];
+    b[3] -= m1 * a[4];
+    m2 = c[0] * iv;
+    c[1] -= m2 * a[3];
+    c[2] -= m2 * a[4];
+  };
+  put_lo(0, 0, 0.0, 0.0);
+  double w0[5] = {0.0, 0.0, 1.0, 0.0, 0.0}, w1[5], w2[5];
+  ahead(1);
+  interior(w1);
+  ahead(2);
+  interior(w2);
+  ahead(3);
+  // rows k whose incoming row k+3 is an interior one
+  auto step = [&](int k, double (&a)[5], double (&b)[5], double (&c)[5]) {
+    double iv, m1, m2;
+    eliminate(a, b, c, iv, m1, m2);
+    store_row(iv, a[3], a[4], m1, m2);
+    interior(a);
+    ahead(k + 4);
+  };
+  int k = 0;
+  for (; k + 2 <= my - 5; k += 3) {
+    step(k, w0, w1, w2);
+    step(k + 1, w1, w2, w0);
+    step(k + 2, w2, w0, w1);
+  }
+  // the last rows: the incoming row is an interior one, the identity (row
+  // my-1) or none
+  for (; k < my; ++k) {
+    double iv, m1, m2;
+    eliminate(w0, w1, w2, iv, m1, m2);
+    store_row(iv, k + 1 < my ? w0[3] : 0.0, k + 2 < my ? w0[4] : 0.0, k + 1 < my ? m1 : 0.0,
+              k + 2 < my ? m2 : 0.0);
+    const int j = k + 3;
+    double w3[5];
+    if (j < my - 1) {
+      ahead(j);
+      interior(w3);
+    } else {
+#pragma unroll
+      for (int d = 0; d < 5; ++d) w3[d] = d == 2 && j == my - 1 ? 1.0 : 0.0;
+    }
+#pragma unroll
+    for (int d = 0; d < 5; ++d) { w0[d] = w1[d]; w1[d] = w2[d]; w2[d] = w3[d]; }
+  }
+  for (; k < WAVE * M; ++k) store_row(0.0, 0.0, 0.0, 0.0, 0.0);
 }
 
 int launch_helm_factor(const double* dt21, const double* dt22, int my, int M,
-                       const double* shifts, int nsys, double* lu, hipStream_t st) {
+                       const double* shifts, double shift, int nsys, double* lu,
+                       hipStream_t st) {
   if (nsys <= 0) return 0;
-  hipLaunchKernelGGL(k_helm_factor, dim3((nsys + 63) / 64), dim3(64), 0, st, dt21, dt22,
-                     my, M, shifts, nsys, lu);
+  hipLaunchKernelGGL(k_helm_factor, dim3((nsys + 63) / 64), dim3(64), 10 * (size_t)my * 8, st, dt21, dt22,
+                     my, M, shifts, shift, nsys, lu);
   return (int)hipGetLastError();
 }
 

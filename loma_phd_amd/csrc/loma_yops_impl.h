@@ -47,60 +47,76 @@ __device__ __forceinline__ double wave_sum(double v) {
 // ------------------------------------------------------------------------
 // Neumann (solvepsi) pieces
 // ------------------------------------------------------------------------
-// dot products of a complex column with the boundary-derivative functionals
-// w0 (d/dy at row 0) and w1 (d/dy at row my-1): out = {w0.re, w0.im, w1.re,
-// w1.im}.
-template <int M>
-__device__ __forceinline__ void bd_dots(const YTab& T, int lane, const double (&x)[2][M],
-                                        double (&out)[4]) {
+// dot products of real columns with the boundary-derivative functionals w0
+// (d/dy at row 0) and w1 (d/dy at row my-1): out[n] = w0.x_n, out[NC+n] =
+// w1.x_n.
+template <int M, int NC>
+__device__ __forceinline__ void bd_dots(const YTab& T, int lane, const double (&x)[NC][M],
+                                        double (&out)[2 * NC]) {
   RowStream<double, 2, M> w;
-  double s0r = 0.0, s0i = 0.0, s1r = 0.0, s1i = 0.0;
+  double s[2 * NC];
+#pragma unroll
+  for (int q = 0; q < 2 * NC; ++q) s[q] = 0.0;
 #pragma unroll
   for (int t = 0; t < M; ++t) {
     w.up(ytab<M>(T, YT_WBD, lane), t);
     const double a = w(t, 0), b = w(t, 1);
-    s0r += a * x[0][t];
-    s0i += a * x[1][t];
-    s1r += b * x[0][t];
-    s1i += b * x[1][t];
+#pragma unroll
+    for (int n = 0; n < NC; ++n) {
+      s[n] += a * x[n][t];
+      s[NC + n] += b * x[n][t];
+    }
   }
-  out[0] = wave_sum(s0r);
-  out[1] = wave_sum(s0i);
-  out[2] = wave_sum(s1r);
-  out[3] = wave_sum(s1i);
+#pragma unroll
+  for (int q = 0; q < 2 * NC; ++q) out[q] = wave_sum(s[q]);
+}
+
+// Particular and homogeneous solutions of (dt22 - rK dt21) x = . for one
+// factored matrix in one pair of sweeps: x[0], x[1] = the zero-Dirichlet
+// solution for dt21 f, x[2] = LU^{-1} e_0, x[3] = LU^{-1} e_{my-1}, and their
+// boundary derivatives d (bd_dots).
+template <int M>
+__device__ __forceinline__ void solve_with_ends(const YTab& T, const double* lu, int lane,
+                                                const double (&f)[2][M], double (&x)[4][M],
+                                                double (&d)[8]) {
+  {
+    double v[2][M];
+    bmatvec<M, 2, 2>(ytab<M>(T, YT_A2, lane), lane, f, v);
+    const int r0 = lane * M;
+#pragma unroll
+    for (int t = 0; t < M; ++t) {
+      const bool bot = r0 + t == 0, top = r0 + t == T.my - 1;
+      x[0][t] = bot || top ? 0.0 : v[0][t];
+      x[1][t] = bot || top ? 0.0 : v[1][t];
+      x[2][t] = bot ? 1.0 : 0.0;
+      x[3][t] = top ? 1.0 : 0.0;
+    }
+  }
+  op_fence();
+  lsolve<M, 2, 4>(lu_lo<M>(lu, lane), lane, x);
+  op_fence();
+  usolve<M, 2, 4>(lu_up<M>(lu, lane), lane, x);
+  op_fence();
+  bd_dots<M, 4>(T, lane, x, d);
 }
 
 // v solving (dt22 - rK dt21) v = dt21 f in the interior with dv/dy = 0 at
-// both ends (solvepsi, laps.f:580-726).  The reference adds two homogeneous
-// Dirichlet solutions h1, h2 to the zero-Dirichlet particular solution; here
-// the boundary derivatives of h1, h2 are per-class constants
-// bc = {w0.h1, w0.h2, w1.h1, w1.h2}, the particular solution's are two dot
-// products, and the combination is a second Dirichlet solve whose end values
-// are the 2x2 solution (same linear algebra, half the live columns).
+// both ends (solvepsi, laps.f:580-726): the zero-Dirichlet solution plus the
+// two homogeneous ones with the coefficients that clear its end derivatives.
 template <int M>
-__device__ __forceinline__ void solve_neumann(const YTab& T, const double* lu,
-                                              const double* bc, int lane,
+__device__ __forceinline__ void solve_neumann(const YTab& T, const double* lu, int lane,
                                               const double (&f)[2][M], double (&v)[2][M]) {
-  op_helm<M, 2>(T, lu, lane, f, v);
-  double dp[4];
-  bd_dots<M>(T, lane, v, dp);
-  const double a11 = bc[0], a12 = bc[1], a21 = bc[2], a22 = bc[3];
+  double x[4][M], d[8];
+  solve_with_ends<M>(T, lu, lane, f, x, d);
+  const double a11 = d[2], a12 = d[3], a21 = d[6], a22 = d[7];
   const double det = a11 * a22 - a12 * a21;
-  const double cr1 = (-dp[0] * a22 + a12 * dp[2]) / det;
-  const double cr2 = (-a11 * dp[2] + a21 * dp[0]) / det;
-  const double ci1 = (-dp[1] * a22 + a12 * dp[3]) / det;
-  const double ci2 = (-a11 * dp[3] + a21 * dp[1]) / det;
-  // second solve with Dirichlet end values (c1, c2)
-  bmatvec<M, 2, 2>(ytab<M>(T, YT_A2, lane), lane, f, v);
-  const int r0 = lane * M;
 #pragma unroll
-  for (int t = 0; t < M; ++t) {
-    const int r = r0 + t;
-    if (r == 0) { v[0][t] = cr1; v[1][t] = ci1; }
-    if (r == T.my - 1) { v[0][t] = cr2; v[1][t] = ci2; }
+  for (int n = 0; n < 2; ++n) {
+    const double c1 = (-d[n] * a22 + a12 * d[4 + n]) / det;
+    const double c2 = (-a11 * d[4 + n] + a21 * d[n]) / det;
+#pragma unroll
+    for (int t = 0; t < M; ++t) v[n][t] = x[n][t] + (c1 * x[2][t] + c2 * x[3][t]);
   }
-  lsolve<M, 2, 2>(lu_lo<M>(lu, lane), lane, v);
-  usolve<M, 2, 2>(lu_up<M>(lu, lane), lane, v);
 }
 
 // per-class Neumann constants: h1 = LU^{-1} e_0, h2 = LU^{-1} e_{my-1};
@@ -131,7 +147,7 @@ __global__ __launch_bounds__(256) void k_helm_bc(YTab T, const double* lu, int l
     }
   }
   double d[4];
-  bd_dots<M>(T, lane, h, d);  // {w0.h1, w0.h2, w1.h1, w1.h2}
+  bd_dots<M, 2>(T, lane, h, d);  // {w0.h1, w0.h2, w1.h1, w1.h2}
   if (lane == 0) {
     bc[(size_t)wave * 4 + 0] = d[0];
     bc[(size_t)wave * 4 + 1] = d[1];
@@ -164,7 +180,7 @@ __global__ __launch_bounds__(256) void k_dy(YTab T, const double2* u, double2* d
 // mode 2: Dirichlet Helmholtz (visc kernel), no derivative output
 template <int M>
 __global__ __launch_bounds__(256) void k_lapvdvhom(YTab T, const double* lu, int lu_stride,
-                                                   const double* bc, const double2* phi,
+                                                   const double2* phi,
                                                    double2* v, double2* dv,
                                                    const double* rK, int ncols, int mode) {
   LOMA_STAGE(M);
@@ -179,7 +195,7 @@ __global__ __launch_bounds__(256) void k_lapvdvhom(YTab T, const double* lu, int
 #pragma unroll
     for (int t = 0; t < M; ++t) x[0][t] = x[1][t] = 0.0;
   } else if (mode == 1) {
-    solve_neumann<M>(T, L, bc + (size_t)wave * 4, lane, f, x);
+    solve_neumann<M>(T, L, lane, f, x);
   } else {
     op_helm<M, 2>(T, L, lane, f, x);
   }
@@ -201,13 +217,13 @@ __global__ __launch_bounds__(256) void k_lapvdvhom(YTab T, const double* lu, int
 //   v     = (D2 - rk2)^{-1} phi with the Robin rows sqrt(rk2) v - dv/dy = 0
 //     (bottom) and sqrt(rk2) v + dv/dy = 0 (top): of the reference's 4x4
 //     system the phi rows fix the phi coefficients to zero and leave this
-//     2x2 for the end values (c3, c4) of v, solved here in closed form;
+//     2x2 for the end values (c3, c4) of v, solved here in closed form from
+//     the end derivatives of the rk2 homogeneous solutions;
 //   vor = dalbe omega + dtri vorwk + dtxi v_in, phi likewise with dvdy_in
 //     (dalbe != 0), else omega and phi; v = dvdy = 0 when rk2 = 0.
 template <int M>
 __global__ __launch_bounds__(256) void k_visc(YTab T, const double* lu1, const double* lu2,
-                                              int lu_stride, const double* bc2,
-                                              double2* vorwk, double2* vor, double2* phi,
+                                              int lu_stride, double2* vorwk, double2* vor, double2* phi,
                                               double2* v, double2* dvdy, double2* phiwk,
                                               const double* rk2, double dalbe, double dtri,
                                               double dtxi, int ncols) {
@@ -261,27 +277,21 @@ __global__ __launch_bounds__(256) void k_visc(YTab T, const double* lu1, const d
     return;
   }
   {
-    double vp[2][M], dp[4];
-    op_helm<M, 2>(T, L2, lane, x, vp);
-    bd_dots<M>(T, lane, vp, dp);  // {w0.vp re, im, w1.vp re, im}
-    const double* bc = bc2 + (size_t)col * 4;
-    const double k = sqrt(k2);
-    const double m11 = k - bc[0], m12 = -bc[1], m21 = bc[2], m22 = k + bc[3];
-    const double det = m11 * m22 - m12 * m21;
-    const double c3r = (dp[0] * m22 + m12 * dp[2]) / det;
-    const double c4r = (-m11 * dp[2] - m21 * dp[0]) / det;
-    const double c3i = (dp[1] * m22 + m12 * dp[3]) / det;
-    const double c4i = (-m11 * dp[3] - m21 * dp[1]) / det;
-    // second Dirichlet solve with end values (c3, c4)
-    bmatvec<M, 2, 2>(ytab<M>(T, YT_A2, lane), lane, x, vp);
+    double vp[2][M];
+    {
+      double q[4][M], d[8];
+      solve_with_ends<M>(T, L2, lane, x, q, d);
+      const double k = sqrt(k2);
+      const double m11 = k - d[2], m12 = -d[3], m21 = d[6], m22 = k + d[7];
+      const double det = m11 * m22 - m12 * m21;
 #pragma unroll
-    for (int t = 0; t < M; ++t) {
-      const int r = r0 + t;
-      if (r == 0) { vp[0][t] = c3r; vp[1][t] = c3i; }
-      if (r == my - 1) { vp[0][t] = c4r; vp[1][t] = c4i; }
+      for (int n = 0; n < 2; ++n) {
+        const double c3 = (d[n] * m22 + m12 * d[4 + n]) / det;
+        const double c4 = (-m11 * d[4 + n] - m21 * d[n]) / det;
+#pragma unroll
+        for (int t = 0; t < M; ++t) vp[n][t] = q[n][t] + (c3 * q[2][t] + c4 * q[3][t]);
+      }
     }
-    lsolve<M, 2, 2>(lu_lo<M>(L2, lane), lane, vp);
-    usolve<M, 2, 2>(lu_up<M>(L2, lane), lane, vp);
     store_col<M>(v + o, my, lane, st, vp);
     op_dy1<M, 2>(T, lane, vp, f);
     store_col<M>(dvdy + o, my, lane, st, f);
@@ -514,27 +524,6 @@ __global__ __launch_bounds__(256, 3) void k_phaseC32_batch(const PhaseArgs* __re
 // for two modes.  The Neumann combination is v + c1 h1 + c2 h2 with h1, h2
 // from the class table (the second Dirichlet solve of solvepsi, laps.f:
 // 700-726, by linearity).  The class with kx = kz = 0 is the 00 mode alone.
-template <int M>
-__device__ __forceinline__ void bd_dots4(const YTab& T, int lane, const double (&x)[4][M],
-                                         double (&out)[8]) {
-  RowStream<double, 2, M> w;
-  double s[8];
-#pragma unroll
-  for (int q = 0; q < 8; ++q) s[q] = 0.0;
-#pragma unroll
-  for (int t = 0; t < M; ++t) {
-    w.up(ytab<M>(T, YT_WBD, lane), t);
-    const double a = w(t, 0), b = w(t, 1);
-#pragma unroll
-    for (int n = 0; n < 4; ++n) {
-      s[n] += a * x[n][t];
-      s[4 + n] += b * x[n][t];
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < 8; ++q) out[q] = wave_sum(s[q]);
-}
-
 template <int M, typename TS>
 __global__ __launch_bounds__(256) void k_phaseC2(PhaseArgs a) {
   const int bx = blockIdx.x;
@@ -783,21 +772,21 @@ int launch_dy_m(int order, const YTab& T, const double* u, double* du, int ncols
   return (int)hipGetLastError();
 }
 template <int M>
-int launch_lapvdvhom_m(const YTab& T, const double* lu, int lu_stride, const double* bc,
-                       const double* phi, double* v, double* dv, const double* rK, int ncols,
+int launch_lapvdvhom_m(const YTab& T, const double* lu, int lu_stride, const double* phi,
+                       double* v, double* dv, const double* rK, int ncols,
                        int mode, hipStream_t st) {
   dim3 g((ncols + 3) / 4), b(256);
-  hipLaunchKernelGGL((k_lapvdvhom<M>), g, b, 0, st, T, lu, lu_stride, bc,
+  hipLaunchKernelGGL((k_lapvdvhom<M>), g, b, 0, st, T, lu, lu_stride,
                      (const double2*)phi, (double2*)v, (double2*)dv, rK, ncols, mode);
   return (int)hipGetLastError();
 }
 template <int M>
 int launch_visc_m(const YTab& T, const double* lu1, const double* lu2, int lu_stride,
-                  const double* bc2, double* vorwk, double* vor, double* phi, double* v,
+                  double* vorwk, double* vor, double* phi, double* v,
                   double* dvdy, double* phiwk, const double* rk2, double dalbe, double dtri,
                   double dtxi, int ncols, hipStream_t st) {
   dim3 g((ncols + 3) / 4), b(256);
-  hipLaunchKernelGGL((k_visc<M>), g, b, 0, st, T, lu1, lu2, lu_stride, bc2, (double2*)vorwk,
+  hipLaunchKernelGGL((k_visc<M>), g, b, 0, st, T, lu1, lu2, lu_stride, (double2*)vorwk,
                      (double2*)vor, (double2*)phi, (double2*)v, (double2*)dvdy,
                      (double2*)phiwk, rk2, dalbe, dtri, dtxi, ncols);
   return (int)hipGetLastError();
@@ -870,15 +859,15 @@ namespace loma {
 #define LOMA_INSTANTIATE_M(MV)                                                        \
   template int launch_dy_m<MV>(int, const YTab&, const double*, double*, int, hipStream_t); \
   template int launch_lapvdvhom_m<MV>(const YTab&, const double*, int, const double*,     \
-                                      const double*, double*, double*, const double*, int, \
-                                      int, hipStream_t);                                  \
+                                      double*, double*, const double*, int, int,          \
+                                      hipStream_t);                                       \
   template int launch_helm_bc_m<MV>(const YTab&, const double*, int, double*, double*,    \
                                     int, hipStream_t);                                    \
   template int launch_inty8_m<MV>(const YTab&, const double*, double*, hipStream_t);      \
   template int launch_visc_m<MV>(const YTab&, const double*, const double*, int,          \
-                                 const double*, double*, double*, double*, double*,       \
-                                 double*, double*, const double*, double, double, double, \
-                                 int, hipStream_t);                                       \
+                                 double*, double*, double*, double*, double*, double*,    \
+                                 const double*, double, double, double, int,              \
+                                 hipStream_t);                                            \
   template int launch_phase_m<MV>(int, bool, const PhaseArgs&, hipStream_t);              \
   template int launch_phase_batch_m<MV>(int, bool, const PhaseArgs*, const int*, int, int,  \
                                         hipStream_t);                                     \
