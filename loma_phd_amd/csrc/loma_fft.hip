@@ -13,6 +13,7 @@
 // 8/4/2/3/5 (Govindaraju et al., SC'08 formulation), one workgroup per tile.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -975,67 +976,65 @@ struct XRow {
     twiddle_pow<E>(w, tw.inv2, +1);
     dft_r<E, T, T2>(w, +1);
   }
-  __device__ static __forceinline__ void forward(T2* A, int jl, const Tw& tw, T2 (&w)[E]) {
-    dft_r<E, T, T2>(w, -1);
+  // Transform of sign s (first twiddles of sign -1) of the row whose entries
+  // jl + RL r are in w; the results stay in registers, v[q][r] = entry
+  // jl + RL q + NLAST r of the row (lanes of q with jl + RL q < NLAST).
+  static constexpr int RLAST = E == 8 ? (R0 > 1 ? R0 : 8) : RB;  // radix of the last pass
+  static constexpr int NLAST = N / RLAST;
+  __device__ static __forceinline__ bool last_on(int jl, int q) {
+    return NLAST % RL == 0 || jl + RL * q < NLAST;
+  }
+  // position of entry jl + RL q + NLAST r (NLAST is a multiple of 8)
+  __device__ static __forceinline__ int last_at(int jl, int q, int r) {
+    return li(jl) + RL / 8 * 9 * q + NLAST / 8 * 9 * r;
+  }
+  __device__ static __forceinline__ void row_fft(T2* A, int jl, const Tw& tw, int s, T2 (&w)[E],
+                                                 T2 (&v)[NL][RLAST]) {
+    dft_r<E, T, T2>(w, s);
 #pragma unroll
     for (int r = 0; r < E; ++r) A[E == 8 ? 9 * jl + r : li(6 * jl + r)] = w[r];
     wave_sync();
-    if constexpr (E == 8) {
+    const bool on = E == 8 || jl < N / 8;
+    T2 u[8];
+    if (on) {
 #pragma unroll
-      for (int r = 0; r < 8; ++r) w[r] = A[at(jl, r)];
-      twiddle_pow<8>(w, tw.fwd1, -1);
-      dft8<T, T2>(w, -1);
-      wave_sync();
-      const int o = li(jl / 8 * 64 + jl % 8);
+      for (int r = 0; r < 8; ++r) u[r] = A[E == 8 ? at(jl, r) : li(jl + r * (N / 8))];
+    }
+    if constexpr (E == 8 && R0 == 1) {
+      twiddle_pow<8>(u, tw.fwd2[0], s);
+      dft8<T, T2>(u, s);
 #pragma unroll
-      for (int r = 0; r < 8; ++r) A[o + 9 * r] = w[r];
-      if constexpr (R0 > 1) {
-        wave_sync();
-#pragma unroll
-        for (int q = 0; q < NL; ++q)
-#pragma unroll
-          for (int r = 0; r < R0; ++r) w[q * R0 + r] = A[li(jl) + RL / 8 * 9 * q + 72 * r];
-#pragma unroll
-        for (int q = 0; q < NL; ++q) {
-          twiddle_pow<R0>(w + q * R0, tw.fwd2[q], -1);
-          dft_r<R0, T, T2>(w + q * R0, -1);
-        }
-        wave_sync();
-#pragma unroll
-        for (int q = 0; q < NL; ++q)
-#pragma unroll
-          for (int r = 0; r < R0; ++r) A[li(jl) + RL / 8 * 9 * q + 72 * r] = w[q * R0 + r];
-      }
+      for (int r = 0; r < 8; ++r) v[0][r] = u[r];
     } else {
-      const bool on = jl < N / 8;
-      T2 u[8];
-      if (on) {
-#pragma unroll
-        for (int r = 0; r < 8; ++r) u[r] = A[li(jl + r * (N / 8))];
-      }
       wave_sync();
       if (on) {
-        twiddle_pow<8>(u, tw.fwd1, -1);
-        dft8<T, T2>(u, -1);
-        const int o = jl / 6 * 48 + jl % 6;
+        twiddle_pow<8>(u, tw.fwd1, s);
+        dft8<T, T2>(u, s);
+        const int o = jl / E * (8 * E) + jl % E;
 #pragma unroll
-        for (int r = 0; r < 8; ++r) A[li(o + 6 * r)] = u[r];
+        for (int r = 0; r < 8; ++r) A[E == 8 ? li(o) + 9 * r : li(o + 6 * r)] = u[r];
       }
       wave_sync();
-      // in place: an item's outputs are its inputs' entries
 #pragma unroll
       for (int q = 0; q < NL; ++q)
-        if (48 % RL == 0 || jl + RL * q < 48) {
-          T2 v[RB];
-          const int o = li(jl) + RL / 8 * 9 * q;
+        if (last_on(jl, q)) {
 #pragma unroll
-          for (int r = 0; r < RB; ++r) v[r] = A[o + 54 * r];
-          twiddle_pow<RB>(v, tw.fwd2[q], -1);
-          dft_r<RB, T, T2>(v, -1);
-#pragma unroll
-          for (int r = 0; r < RB; ++r) A[o + 54 * r] = v[r];
+          for (int r = 0; r < RLAST; ++r) v[q][r] = A[last_at(jl, q, r)];
+          twiddle_pow<RLAST>(v[q], tw.fwd2[q], s);
+          dft_r<RLAST, T, T2>(v[q], s);
         }
     }
+  }
+  __device__ static __forceinline__ void forward(T2* A, int jl, const Tw& tw, T2 (&w)[E]) {
+    T2 v[NL][RLAST];
+    row_fft(A, jl, tw, -1, w, v);
+    wave_sync();
+#pragma unroll
+    for (int q = 0; q < NL; ++q)
+      if (last_on(jl, q)) {
+#pragma unroll
+        for (int r = 0; r < RLAST; ++r) A[last_at(jl, q, r)] = v[q][r];
+      }
   }
   // Hermitian unpacking into a field, scaled by 1/N (lines past my go to the
   // row's padding, which is never read, or are dropped)
@@ -1080,24 +1079,58 @@ __attribute__((amdgpu_waves_per_eu(2))) void k_xrow_batch(
 #include "loma_xrow_body.inc"
 }
 
-// fourz on standalone rows (FFTPACK convention), for the per-operator API
+// fourz on standalone rows (FFTPACK convention), for the per-operator API.
+// Lengths of XRow: RL lanes of a wavefront per row, from and to HBM in
+// registers (runs of RL entries), two exchanges through the row's LDS and no
+// workgroup barrier: 87,210 rows of 256 take 143 us, the rate of a copy, where
+// one workgroup a row took 321
+template <int N>
+__global__ __launch_bounds__(256) void k_fourz_row(const double2* __restrict__ tw, double2* c,
+                                                   int nrows, int iopt) {
+  using C = XRow<double, N>;
+  constexpr int RL = C::RL, ROWS = 256 / RL;
+  __shared__ double2 buf[ROWS * C::RS];
+  const int lr = threadIdx.x / RL, jl = threadIdx.x - lr * RL;
+  const long long row = (long long)blockIdx.x * ROWS + lr;
+  if (row >= nrows) return;
+  const typename C::Tw twd = C::twiddles(tw, jl);
+  double2* p = c + row * N + jl;
+  double2 w[C::E], v[C::NL][C::RLAST];
+#pragma unroll
+  for (int r = 0; r < C::E; ++r) w[r] = p[RL * r];
+  C::row_fft(buf + lr * C::RS, jl, twd, iopt < 0 ? -1 : 1, w, v);
+  const double sc = iopt < 0 ? 1.0 / N : 1.0;
+#pragma unroll
+  for (int q = 0; q < C::NL; ++q)
+    if (C::last_on(jl, q)) {
+#pragma unroll
+      for (int r = 0; r < C::RLAST; ++r) {
+        double2 y = v[q][r];
+        y.x *= sc;
+        y.y *= sc;
+        p[RL * q + C::NLAST * r] = y;
+      }
+    }
+}
+// other lengths: as many rows a workgroup as fill its threads, run-time plan
 __global__ __launch_bounds__(256) void k_fourz(FftPlan pl, const double2* tw, double2* c,
-                                               int nrows, int iopt) {
+                                               int nrows, int iopt, int per) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int N = pl.n;
   double2* A = (double2*)smem;
-  double2* B = A + lds_entries(N);
-  const int row = blockIdx.x;
-  if (row >= nrows) return;
-  for (int it = threadIdx.x; it < N; it += blockDim.x) A[lds_i(it)] = c[(size_t)row * N + it];
+  double2* B = A + lds_entries(N * per);
+  const long long row0 = (long long)blockIdx.x * per;
+  const int nr = (int)min((long long)per, nrows - row0);
+  double2* p = c + row0 * N;
+  for (int it = threadIdx.x; it < nr * N; it += blockDim.x) A[lds_i(it)] = p[it];
   __syncthreads();
-  double2* R = fft_rows<double, double2>(A, B, N, N, 1, pl, tw, iopt < 0 ? -1 : 1);
+  double2* R = fft_rows<double, double2>(A, B, N, N, nr, pl, tw, iopt < 0 ? -1 : 1);
   const double sc = iopt < 0 ? 1.0 / N : 1.0;
-  for (int it = threadIdx.x; it < N; it += blockDim.x) {
+  for (int it = threadIdx.x; it < nr * N; it += blockDim.x) {
     double2 v = R[lds_i(it)];
     v.x *= sc;
     v.y *= sc;
-    c[(size_t)row * N + it] = v;
+    p[it] = v;
   }
 }
 
@@ -1269,10 +1302,26 @@ int launch_xline_batch(bool fp32, const FftArgs& proto, const FftArgs* args, con
 int launch_fourz(const FftPlan& pl, const double2* tw, double2* c, int nrows, int iopt,
                  hipStream_t st) {
   if (nrows <= 0) return 0;
-  hipLaunchKernelGGL(k_fourz, dim3(nrows), dim3(256), (size_t)2 * lds_entries(pl.n) * 16, st, pl, tw, c,
-                     nrows, iopt);
+  switch (pl.n) {
+#define LOMA_FOURZ_ROW(n)                                                                       \
+    case n: {                                                                                   \
+      constexpr int rows = 256 / XRow<double, n>::RL;                                           \
+      hipLaunchKernelGGL((k_fourz_row<n>), dim3((nrows + rows - 1) / rows), dim3(256), 0, st, tw, \
+                         c, nrows, iopt);                                                       \
+      break;                                                                                    \
+    }
+    LOMA_FOURZ_ROW(64) LOMA_FOURZ_ROW(96) LOMA_FOURZ_ROW(128) LOMA_FOURZ_ROW(192)
+    LOMA_FOURZ_ROW(256) LOMA_FOURZ_ROW(384) LOMA_FOURZ_ROW(512)
+#undef LOMA_FOURZ_ROW
+    default: {
+      // a butterfly's radix is at most 8: 2048 entries keep 256 threads busy
+      // (both buffers 64 KiB); longer rows go one to a workgroup
+      const int per = std::max(1, 2048 / pl.n);
+      hipLaunchKernelGGL(k_fourz, dim3((nrows + per - 1) / per), dim3(256),
+                         (size_t)2 * lds_entries(pl.n * per) * 16, st, pl, tw, c, nrows, iopt, per);
+    }
+  }
   return (int)hipGetLastError();
 }
-
 
 }  // namespace loma
