@@ -43,6 +43,9 @@ struct FftPlan {
   int n;
   int npass;
   int rad[10];
+  // reciprocals of a pass's items per row (n / radix) and sub-length (the
+  // product of the radices before it), for fast_div
+  float inb[10], ins[10];
 };
 FftPlan make_plan(int n);
 
