@@ -1331,8 +1331,10 @@ int launch_fourz(const FftPlan& pl, const double2* tw, double2* c, int nrows, in
 #undef LOMA_FOURZ_ROW
     default: {
       // a butterfly's radix is at most 8: 2048 entries keep 256 threads busy
-      // (both buffers 64 KiB); longer rows go one to a workgroup
-      const int per = std::max(1, 2048 / pl.n);
+      // (both buffers 72 KiB); longer rows go one to a workgroup.  Few rows are
+      // spread over the chip first, four workgroups to a CU: 734 rows of 216 take
+      // 20 us nine to a workgroup and 17 us one to a workgroup
+      const int per = std::max(1, std::min(2048 / pl.n, nrows / 1024));
       hipLaunchKernelGGL(k_fourz, dim3((nrows + per - 1) / per), dim3(256),
                          (size_t)2 * lds_entries(pl.n * per) * 16, st, pl, tw, c, nrows, iopt, per);
     }
