@@ -272,7 +272,7 @@ int loma_visc(loma_run *run, float *vorwk, float *vor, float *phi, float *v,
  * without pivoting (bandec, cfdiff.f:977) and the two triangular sweeps
  * (banbks, cfdiff.f:954), FP64.  The solution goes to x (double,
  * interleaved); x may be NULL for a double rhs, which is then overwritten.
- * Device pointers; stream may be NULL.  Scratch of n*5*nsys doubles is kept
+ * Device pointers; stream may be NULL.  Scratch of n*4*nsys doubles is kept
  * per device and grown on demand. */
 int loma_band5_solve_dev(const double *band, void *rhs, double *x, int n,
                          int nsys, int rhs_fp32, void *stream);

@@ -2387,7 +2387,7 @@ int loma_band5_solve_dev(const double* band, void* rhs, double* x, int n, int ns
   if (nsys == 0) return LOMA_OK;
   int dev = 0;
   HIPCHK(hipGetDevice(&dev));
-  const size_t need = (size_t)n * 5 * nsys * sizeof(double);
+  const size_t need = (size_t)n * 4 * nsys * sizeof(double);
   std::lock_guard<std::mutex> lk(g_band_mu);
   if ((int)g_band_scr.size() <= dev) g_band_scr.resize(dev + 1, {nullptr, 0});
   auto& e = g_band_scr[dev];
