@@ -229,6 +229,7 @@ int launch_xline(bool fp32, const FftArgs& a, hipStream_t st);
 int launch_zfft_fwd(bool fp32, const FftArgs& a, hipStream_t st);
 int launch_fourz(const FftPlan& pl, const double2* tw, double2* c, int nrows, int iopt,
                  hipStream_t st);
+int launch_narrow(const double* src, float* dst, size_t n, hipStream_t st);
 int launch_band5(const double* band, const void* rhs, double* x, double* scratch, int n,
                  int nsys, int rhs_fp32, hipStream_t st);
 

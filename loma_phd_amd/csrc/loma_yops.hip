@@ -3,6 +3,8 @@
 // instantiated one M per translation unit (loma_yops_m<M>.hip).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "loma_kernels.h"
 
 namespace loma {
@@ -363,6 +365,27 @@ int launch_finish_step(DevScalars* sc, RunConst rc, int icfl, const double* cflp
     return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL(k_finish_step, dim3(1), dim3(FINISH_THREADS), 0, st, sc, rc, icfl, cflp,
                      ntile);
+  return (int)hipGetLastError();
+}
+
+// n doubles (an even number) rounded to floats in host memory: the link bounds
+// it, so few workgroups do
+__global__ __launch_bounds__(256) void k_narrow(const double2* __restrict__ src,
+                                                float* __restrict__ dst, size_t n) {
+  const size_t step = (size_t)gridDim.x * 256;
+  for (size_t q = blockIdx.x * 256 + threadIdx.x; q < n / 4; q += step) {
+    const double2 a = src[2 * q], b = src[2 * q + 1];
+    ((float4*)dst)[q] = float4{(float)a.x, (float)a.y, (float)b.x, (float)b.y};
+  }
+  if (n % 4 && blockIdx.x == 0 && threadIdx.x == 0) {
+    const double2 a = src[n / 2 - 1];
+    ((float2*)dst)[n / 2 - 1] = float2{(float)a.x, (float)a.y};
+  }
+}
+int launch_narrow(const double* src, float* dst, size_t n, hipStream_t st) {
+  if (!n) return 0;
+  const unsigned g = (unsigned)std::min<size_t>(128, (n / 4 + 255) / 256 + 1);
+  hipLaunchKernelGGL(k_narrow, dim3(g), dim3(256), 0, st, (const double2*)src, dst, n);
   return (int)hipGetLastError();
 }
 
