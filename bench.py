@@ -130,7 +130,7 @@ def algorithmic_bytes(run, with_z: bool):
     S, W, P = run.S, run.W, run.P
     es = 8 if run.precision == 1 else 16
     z = 1 if with_z else 0
-    nin, nout = (12, 12) if with_z else (8, 11)
+    nin, nout = (11, 11) if with_z else (7, 10)
     k = {
         # reads phi, ten13, vor, ten12, psi, T (+Z); writes phi, vor; writes
         # the transform inputs

@@ -1066,10 +1066,11 @@ static int enqueue_substep(loma_run* r, int rkstep, int icfl) {
   if (stats) LCHK(launch_stats(r->M, r->fp32, 1, stats_args(r), st));
   FftArgs fa = fft_args(r, rkstep, (rkstep == 1 && icfl) ? 1 : 0);
   fa.stat_rho = stats ? r->st_rho : nullptr;
-  fa.nfields = r->with_z ? 12 : 8;
+  fa.out_rvv = stats ? 1 : 0;
+  fa.nfields = xf_inputs(fa);
   PROF(KC_ZINV, launch_zfft_inv(r->fp32, fa, st));
   PROF(KC_XLINE, launch_xline(r->fp32, fa, st));
-  fa.nfields = r->with_z ? 12 : 11;
+  fa.nfields = xf_outputs(fa);
   PROF(KC_ZFWD, launch_zfft_fwd(r->fp32, fa, st));
   PROF(KC_PHASEC, launch_phaseC(r->M, r->fp32, pa, st));
   PROF(KC_PHASEC2, launch_phaseC2(r->M, r->fp32, pa, st));
@@ -1109,9 +1110,9 @@ static int time_launch(loma_run* r, int which, float* best_ms) {
     HIPCHK(hipEventRecord(a, r->stream));
     int e = 0;
     if (which == 0) {
-      fa.nfields = r->with_z ? 12 : 8;
+      fa.nfields = xf_inputs(fa);
       e = launch_zfft_inv(r->fp32, fa, r->stream);
-      fa.nfields = r->with_z ? 12 : 11;
+      fa.nfields = xf_outputs(fa);
       if (!e) e = launch_zfft_fwd(r->fp32, fa, r->stream);
     } else {
       e = launch_xline(r->fp32, fa, r->stream);
@@ -1257,7 +1258,7 @@ static void ensemble_plan(loma_run* const* runs, int nruns, const std::vector<in
         L.kind = kind; L.which = which;
         L.M = r0->M; L.fp32 = r0->fp32;
         L.proto = fa[0];
-        L.proto.nfields = kind == EnsLaunch::ZINV ? (r0->with_z ? 12 : 8) : (r0->with_z ? 12 : 11);
+        L.proto.nfields = kind == EnsLaunch::ZINV ? xf_inputs(fa[0]) : xf_outputs(fa[0]);
         L.args_off = kind == EnsLaunch::PHASE ? pa_off : fa_off;
         L.first_off = plan.put(first.data(), first.size() * sizeof(int));
         L.nrun = (int)g.size(); L.nblocks = nb;
@@ -2220,10 +2221,11 @@ int loma_foup2(loma_run* r, float* up1, float* up2, float* up3, float* ten11, fl
   HIPCHK(hipMemcpy(r->sc, &s, sizeof(s), hipMemcpyHostToDevice));
   const int do_cfl = rkstep == 1 ? 1 : 0;
   FftArgs fa = fft_args(r, rkstep, do_cfl);
-  fa.nfields = 8;
+  fa.full = 1;
+  fa.nfields = xf_inputs(fa);
   LCHK(launch_zfft_inv(r->fp32, fa, r->stream));
   LCHK(launch_xline(r->fp32, fa, r->stream));
-  fa.nfields = 11;
+  fa.nfields = xf_outputs(fa);
   LCHK(launch_zfft_fwd(r->fp32, fa, r->stream));
   HIPCHK(hipStreamSynchronize(r->stream));
   HIPCHK(hipMemcpy(mean.data(), r->mean_out, mean.size() * 8, hipMemcpyDeviceToHost));

@@ -655,7 +655,7 @@ constexpr int xl_pad() {
 // A (row f*pairs + p = lines j0+2p, j0+2p+1 of field f); no barrier.
 template <typename T, typename T2, int XR, int NF>
 __device__ __forceinline__ void xl_pack_from(const FftArgs& a, const XlIn<T2, XR>* v, T2* A,
-                                             int pairs) {
+                                             int pairs, int dx) {
   constexpr int XP = xl_pad<T>();
   const int N = a.rc.mgalx, np = a.rc.nplanes;
   const int lp = __builtin_ctz(pairs);
@@ -674,8 +674,13 @@ __device__ __forceinline__ void xl_pack_from(const FftArgs& a, const XlIn<T2, XR
       const int it = threadIdx.x + r * XL_THREADS;
       if (it < np * pairs) {
         const int ii = it >> lp, p = it & (pairs - 1);
-        const T2 ca = v[f].a[r], cb = v[f].b[r];
+        T2 ca = v[f].a[r], cb = v[f].b[r];
         const int rb = (f * pairs + p) * RS;
+        if (f == dx) {                // this field times ikx
+          const T kx = (T)(a.rc.alp * ii);
+          ca = T2{-ca.y * kx, ca.x * kx};
+          cb = T2{-cb.y * kx, cb.x * kx};
+        }
         if (ii == 0) {
           // the imaginary part of the kx=0 coefficient is ignored (rft, rftsingle.f:87-91)
           A[lds_i<XP>(rb)] = T2{ca.x, cb.x};
@@ -692,11 +697,11 @@ __device__ __forceinline__ void xl_pack_from(const FftArgs& a, const XlIn<T2, XR
 template <typename T, typename T2, int XR, int NF>
 __device__ __forceinline__ void xl_pack(const FftArgs& a, const T2* __restrict__ src0,
                                         const T2* __restrict__ src1, T2* A, int z, int j0,
-                                        int pairs) {
+                                        int pairs, int dx) {
   XlIn<T2, XR> v[NF];
   xl_fetch<T2, XR>(a, src0, z, j0, pairs, v[0]);
   if constexpr (NF > 1) xl_fetch<T2, XR>(a, src1, z, j0, pairs, v[1]);
-  xl_pack_from<T, T2, XR, NF>(a, v, A, pairs);
+  xl_pack_from<T, T2, XR, NF>(a, v, A, pairs, dx);
 }
 
 // Hermitian unpacking of the transformed pairs in R into fields dst0 (rows
@@ -728,11 +733,13 @@ __device__ __forceinline__ void xl_unpack(const FftArgs& a, const T2* R, T2* __r
   }
 }
 
-// pack, then the inverse FFT.  Returns the buffer holding the physical pairs.
+// pack, then the inverse FFT; the derivative d/dx of field dx (-1: of none).
+// Returns the buffer holding the physical pairs.
 template <typename T, typename T2, int XR, int NF>
 __device__ __forceinline__ T2* xl_inverse(const FftArgs& a, const T2* __restrict__ src0,
-                          const T2* __restrict__ src1, T2* A, T2* B, int z, int j0, int pairs) {
-  xl_pack<T, T2, XR, NF>(a, src0, src1, A, z, j0, pairs);
+                          const T2* __restrict__ src1, T2* A, T2* B, int z, int j0, int pairs,
+                          int dx = -1) {
+  xl_pack<T, T2, XR, NF>(a, src0, src1, A, z, j0, pairs, dx);
   __syncthreads();
   const int N = a.rc.mgalx;
   return fft_rows<T, T2, xl_pad<T>()>(A, B, N, N, NF * pairs, a.plx, (const T2*)a.twx, +1);
@@ -893,6 +900,15 @@ struct XRow {
       const vec q = *(const vec*)((const char*)src + t.off[r]);
       v.a[r] = T2{q[0], q[1]};
       v.b[r] = T2{q[2], q[3]};
+    }
+  }
+  // the coefficients times ikx
+  __device__ static __forceinline__ void ikx(XlIn<T2, XR>& v, int tg, double alp) {
+#pragma unroll
+    for (int r = 0; r < XR; ++r) {
+      const T kx = (T)(alp * ((tg + r * GT) / P));
+      v.a[r] = T2{-v.a[r].y * kx, v.a[r].x * kx};
+      v.b[r] = T2{-v.b[r].y * kx, v.b[r].x * kx};
     }
   }
   // two real lines to one complex row; the imaginary part of the kx = 0

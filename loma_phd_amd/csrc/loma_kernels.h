@@ -121,8 +121,34 @@ struct FftArgs {
   int with_z;
   int J;                     // y rows per z-transform block
   int L;                     // lines per x-line block
+  // x lines: foup2's own fields (dT/dx comes in slot 4; outputs 3, 4, 5 are
+  // ruu, rvv, rww).  Else the step's: dT/dx is ikx T, outputs 3 and 5 are
+  // ruu - rvv and rww - rvv, and rvv goes to slot 4 only with out_rvv
+  int full;
+  int out_rvv;
   int xrow;                  // x lines by k_xrow (xrow_serves)
 };
+
+// The transform fields of a step.  Slot 4 stays empty both ways: dT/dx needs
+// no transform of its own in z (ikx commutes with it), and the step needs
+// rvv only in ruu - rvv and rww - rvv (loma_phaseC_body.inc).  Statistics
+// take the plane sums of ruu, rvv, rww and have rvv as well.  17 fields pass
+// the z transforms instead of 19 (22 instead of 24 with Z): at 512x513x256 a
+// step takes 20.0 instead of 21.5 ms (FP64) and 12.2 instead of 12.9 ms
+// (mixed).  The differences are taken to rvv so that -rK rvv + kx^2 ruu +
+// kz^2 rww, the sum phi needs, is kx^2 (ruu - rvv) + kz^2 (rww - rvv): no
+// larger rounding than the three products had.
+__host__ __device__ inline int xf_inputs(const FftArgs& a) {
+  return (a.with_z ? 12 : 8) - (a.full ? 0 : 1);
+}
+// the slot left out (12: none)
+__host__ __device__ inline int xf_skip_in(const FftArgs& a) { return a.full ? 12 : 4; }
+__host__ __device__ inline int xf_outputs(const FftArgs& a) {
+  return (a.with_z ? 12 : 11) - (a.full || a.out_rvv ? 0 : 1);
+}
+__host__ __device__ inline int xf_skip_out(const FftArgs& a) {
+  return a.full || a.out_rvv ? 12 : 4;
+}
 
 // statistics window (addstats1/2 and the phys2 sums of cross.f): the
 // accumulated columns, in the order of a .sta record, are

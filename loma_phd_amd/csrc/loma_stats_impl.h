@@ -244,7 +244,7 @@ __global__ __launch_bounds__(64) void k_stats_out(StatsArgs a) {
   if (wv == 0) {
     // sum over the plane of rho u_i u_j = mgalx*mgalz times the 00 mode of
     // the transformed product (slot -> column: 3 ruu, 6 ruv, 7 ruw, 4 rvv,
-    // 8 rvw, 5 rww)
+    // 8 rvw, 5 rww; slots 3 and 5 hold ruu - rvv and rww - rvv)
     const double npts = (double)rc.mgalx * (double)rc.mgalz;
     const int slot[6] = {3, 6, 7, 4, 8, 5};
 #pragma unroll 1
@@ -253,6 +253,14 @@ __global__ __launch_bounds__(64) void k_stats_out(StatsArgs a) {
       wave_sync();
       load_col<M>((const T2*)a.spec[slot[q]], my, lane, st, x);
       add_mean<M>(x, lane, my, true, a.mean_out + (size_t)slot[q] * my);
+      if (q == 0 || q == 5) {
+        double v[2][M];
+        wave_sync();
+        load_col<M>((const T2*)a.spec[4], my, lane, st, v);
+        add_mean<M>(v, lane, my, true, a.mean_out + (size_t)4 * my);
+#pragma unroll
+        for (int t = 0; t < M; ++t) x[0][t] += v[0][t];
+      }
 #pragma unroll
       for (int t = 0; t < M; ++t)
         if (r0 + t < my) a.acc[(size_t)(22 + q) * my + r0 + t] += npts * x[0][t];

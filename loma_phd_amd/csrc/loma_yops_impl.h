@@ -457,8 +457,10 @@ __device__ __forceinline__ void scalar_derivs(const PhaseArgs& a, int lane, doub
     }
   }
   if (q_f >= 0) store_spec<M>(sp[q_f] + os, my, lane, st, F, m00, mi + (size_t)q_f * my);
-  mul_i<M>(F, kx, d);
-  store_spec<M>(sp[q_dx] + os, my, lane, st, d, m00, mi + (size_t)q_dx * my);
+  if (q_dx >= 0) {
+    mul_i<M>(F, kx, d);
+    store_spec<M>(sp[q_dx] + os, my, lane, st, d, m00, mi + (size_t)q_dx * my);
+  }
   mul_i<M>(F, kz, d);
   store_spec<M>(sp[q_dz] + os, my, lane, st, d, m00, mi + (size_t)q_dz * my);
   op_dy1<M, 2>(a.T, lane, F, d);
