@@ -190,7 +190,7 @@ static size_t plan_bytes(int mgalx, int my, int mgalz, bool fp32, bool with_z) {
   const size_t P = (size_t)mgalx * my * mgalz, es = fp32 ? 8 : 16;
   const size_t nsp = with_z ? 12 : 11, nst = with_z ? 7 : 6;
   const size_t tw = fp32 ? 8 : 16;
-  size_t b = align256(12 * (size_t)ytab_offset(YT_COUNT, M));  // y tables, FP64 and FP32
+  size_t b = align256(12 * (size_t)ytab_size(M));  // y tables, FP64 and FP32
   b += 2 * align256(8 * 5 * (size_t)my);                       // band copies
   b += align256(8 * nclass) + align256(8 * 5 * R * nclass) + align256(32 * nclass);
   b += align256(8 * 2 * R * nclass);                           // homogeneous solutions
@@ -432,7 +432,7 @@ int loma_init(loma_run** out, int mgalx, int my, int mgalz, const double* y, dou
   }
   // per-row tables and scan compositions at ytab_offset(id, M), the layout
   // the kernels address with constant offsets
-  const size_t tot = ytab_offset(YT_COUNT, M);
+  const size_t tot = ytab_size(M);
   std::vector<double> h(tot, 0.0);
   std::vector<float> h32(tot, 0.0f);
   // entry e of lane l in table `id` (its stream at element `o` holds n
@@ -458,11 +458,18 @@ int loma_init(loma_run** out, int mgalx, int my, int mgalz, const double* y, dou
       if (++t == M) { t = 0; ++l; }
     }
   };
-  put(YT_B1, f.b1, 7, 0); put(YT_A1, f.a1, 7, 0); put(YT_U1, f.inv1, 1, 0);
+  put(YT_A1, f.a1, 7, 0); put(YT_U1, f.inv1, 1, 0);
   put(YT_U1, f.up1, 3, 1); put_lo(YT_LO1, f.lo1); put(YT_FMAP, f.fmap, 1, 0);
   put(YT_B2, f.b2, 5, 0); put(YT_A2, f.a2, 5, 0); put(YT_U2, f.inv2, 1, 0);
   put(YT_U2, f.up2, 2, 1); put_lo(YT_LO2, f.lo2); put(YT_UI, f.invi, 1, 0);
   put(YT_UI, f.upi, 3, 1); put_lo(YT_LOI, f.loi); put(YT_WBD, wbd, 2, 0);
+  // B1: its first and last three rows and an inner one (b1_matvec)
+  for (int q = 0; q < B1_ROWS; ++q)
+    for (int d = 0; d < 7; ++d) {
+      const int j = q < 3 ? q : q < 6 ? my - 6 + q : my / 2;
+      h[ytab_offset(YT_COUNT, M) + q * 7 + d] = f.b1[(size_t)j * 7 + d];
+      h32[ytab_offset(YT_COUNT, M) + q * 7 + d] = (float)f.b1[(size_t)j * 7 + d];
+    }
   // scan compositions, [level][P*P][lane] -> one stream a level
   std::vector<double> hs((size_t)6 * 9 * 64);
   auto scan = [&](int id, bool upper, const double* lo, const double* up, const double* inv) {

@@ -138,6 +138,32 @@ struct RowStream {
   }
 };
 
+// ---- shifts by d lanes ---------------------------------------------------
+// wave_up(v, d): lane l's value is lane l-d's, for l >= d; wave_down(v, d):
+// lane l+d's, for l + d < 64.  d = 1, every halo and carry, brings 0 into the
+// end lane and is a DPP move a word where __shfl_up is an LDS permute and a
+// select.  (All of them in the vector ALU, DPP moves and permlane swaps, was
+// slower: 8 instructions a word for d = 8.)
+template <bool UP>
+__device__ __forceinline__ unsigned lane_next(unsigned x) {
+  return __builtin_amdgcn_update_dpp(0, x, UP ? 0x138 : 0x130, 0xf, 0xf, true);  // wave_shr/shl:1
+}
+template <bool UP, typename V>
+__device__ __forceinline__ V wave_by(V v, int d) {
+  if (d != 1) return UP ? __shfl_up(v, d) : __shfl_down(v, d);
+  if constexpr (sizeof(V) == 4) {
+    return __builtin_bit_cast(V, lane_next<UP>(__builtin_bit_cast(unsigned, v)));
+  } else {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = lane_next<UP>((unsigned)b), hi = lane_next<UP>((unsigned)(b >> 32));
+    return __builtin_bit_cast(V, ((unsigned long long)hi << 32) | lo);
+  }
+}
+template <typename V>
+__device__ __forceinline__ V wave_up(V v, int d) { return wave_by<true>(v, d); }
+template <typename V>
+__device__ __forceinline__ V wave_down(V v, int d) { return wave_by<false>(v, d); }
+
 // ---- wavefront scans of affine maps s_out = A s_in + c -----------------
 template <int P, int NC>
 __device__ __forceinline__ void scan_affine_up(double (&A)[P][P], double (&c)[NC][P],
@@ -148,11 +174,11 @@ __device__ __forceinline__ void scan_affine_up(double (&A)[P][P], double (&c)[NC
 #pragma unroll
     for (int q = 0; q < P; ++q)
 #pragma unroll
-      for (int b = 0; b < P; ++b) Ap[q][b] = __shfl_up(A[q][b], d);
+      for (int b = 0; b < P; ++b) Ap[q][b] = wave_up(A[q][b], d);
 #pragma unroll
     for (int n = 0; n < NC; ++n)
 #pragma unroll
-      for (int q = 0; q < P; ++q) cp[n][q] = __shfl_up(c[n][q], d);
+      for (int q = 0; q < P; ++q) cp[n][q] = wave_up(c[n][q], d);
     if (lane >= d) {
       double cn[NC][P], An[P][P];
 #pragma unroll
@@ -194,11 +220,11 @@ __device__ __forceinline__ void scan_affine_down(double (&A)[P][P], double (&c)[
 #pragma unroll
     for (int q = 0; q < P; ++q)
 #pragma unroll
-      for (int b = 0; b < P; ++b) Ap[q][b] = __shfl_down(A[q][b], d);
+      for (int b = 0; b < P; ++b) Ap[q][b] = wave_down(A[q][b], d);
 #pragma unroll
     for (int n = 0; n < NC; ++n)
 #pragma unroll
-      for (int q = 0; q < P; ++q) cp[n][q] = __shfl_down(c[n][q], d);
+      for (int q = 0; q < P; ++q) cp[n][q] = wave_down(c[n][q], d);
     if (lane + d < WAVE) {
       double cn[NC][P], An[P][P];
 #pragma unroll
@@ -233,7 +259,8 @@ __device__ __forceinline__ void scan_affine_down(double (&A)[P][P], double (&c)[
 
 // ---- unit lower solve: w_r = x_r - sum_{i=1..P} L(r,i) w_{r-i} ------------
 // lo(t, i-1) = L(r0+t, i): multiplier of row r0+t-i into row r0+t.
-template <int M, int P, int NC>
+// KEEP: see lsolve_tab; four columns of eight rows and more leave no room.
+template <int M, int P, int NC, bool KEEP = (NC < 4 || M < 8)>
 __device__ __forceinline__ void lsolve(const TabRef lo, int lane, double (&x)[NC][M]) {
   static_assert(P <= M, "chunk shorter than bandwidth");
   // (1) in place, zero incoming state
@@ -283,20 +310,20 @@ __device__ __forceinline__ void lsolve(const TabRef lo, int lane, double (&x)[NC
   for (int n = 0; n < NC; ++n)
 #pragma unroll
     for (int q = 0; q < P; ++q) {
-      const double v = __shfl_up(c[n][q], 1);
-      s[n][q] = lane == 0 ? 0.0 : v;
+      s[n][q] = wave_up(c[n][q], 1);
     }
-  const TabRef lo2 = relaunder(lo);
   RowStream<double, P, M> L2;
+  TabRef lo2 = lo;
+  if constexpr (!KEEP) lo2 = relaunder(lo);
   double dl[NC][M];
 #pragma unroll
   for (int t = 0; t < M; ++t) {
-    L2.up(lo2, t);
+    if constexpr (!KEEP) L2.up(lo2, t);
 #pragma unroll
     for (int n = 0; n < NC; ++n) dl[n][t] = 0.0;
 #pragma unroll
     for (int i = 1; i <= P; ++i) {
-      const double l = L2(t, i - 1);
+      const double l = KEEP ? L(t, i - 1) : L2(t, i - 1);
 #pragma unroll
       for (int n = 0; n < NC; ++n) {
         const double pv = (t - i >= 0) ? dl[n][t - i] : s[n][i - t - 1];
@@ -310,7 +337,7 @@ __device__ __forceinline__ void lsolve(const TabRef lo, int lane, double (&x)[NC
 
 // ---- upper solve: x_r = (w_r - sum_{d=1..P} U(r,d) x_{r+d}) * inv_r ------
 // up: rows of inv_r, U(r,1..P)
-template <int M, int P, int NC>
+template <int M, int P, int NC, bool KEEP = (NC < 4 || M < 8)>
 __device__ __forceinline__ void usolve(const TabRef up, int lane, double (&x)[NC][M]) {
   RowStream<double, P + 1, M> U;
 #pragma unroll
@@ -359,27 +386,27 @@ __device__ __forceinline__ void usolve(const TabRef up, int lane, double (&x)[NC
   for (int n = 0; n < NC; ++n)
 #pragma unroll
     for (int q = 0; q < P; ++q) {
-      const double v = __shfl_down(c[n][q], 1);
-      s[n][q] = lane == WAVE - 1 ? 0.0 : v;
+      s[n][q] = wave_down(c[n][q], 1);
     }
-  const TabRef up2 = relaunder(up);
   RowStream<double, P + 1, M> U2;
+  TabRef up2 = up;
+  if constexpr (!KEEP) up2 = relaunder(up);
   double dl[NC][M];
 #pragma unroll
   for (int t = M - 1; t >= 0; --t) {
-    U2.down(up2, t);
+    if constexpr (!KEEP) U2.down(up2, t);
 #pragma unroll
     for (int n = 0; n < NC; ++n) dl[n][t] = 0.0;
 #pragma unroll
     for (int d = 1; d <= P; ++d) {
-      const double u = U2(t, d);
+      const double u = KEEP ? U(t, d) : U2(t, d);
 #pragma unroll
       for (int n = 0; n < NC; ++n) {
         const double pv = (t + d < M) ? dl[n][t + d] : s[n][t + d - M];
         dl[n][t] -= u * pv;
       }
     }
-    const double iv = U2(t, 0);
+    const double iv = KEEP ? U(t, 0) : U2(t, 0);
 #pragma unroll
     for (int n = 0; n < NC; ++n) {
       dl[n][t] *= iv;
@@ -396,13 +423,31 @@ __device__ __forceinline__ void usolve(const TabRef up, int lane, double (&x)[NC
 // Only the first `levels` levels are applied: the compositions beyond them
 // are below 1e-22 in max norm (the factors' inverses decay geometrically),
 // checked when the tables are built.
-template <int M, int P, int NC, typename V>
+// A wavefront's table load costs its compute unit 16 cycles whatever its
+// lanes read (7.0-8.8 ns for one to 64 active lanes, one address or 64), and
+// these loads bound the y-operators.  KEEP: the correction sweep takes the
+// factor from the registers of the first sweep instead of loading it again
+// (dt11: 33 of 151 loads at M = 9).  Kernels without room for it (54 and 72
+// registers at M = 9 and P = 3) reload.  PRE: the maps of all levels are
+// loaded before the first sweep, not one memory round trip a level, for a
+// wavefront that others wait for (108 registers at P = 3).
+template <int M, int P, int NC, bool KEEP, bool PRE, typename V>
 __device__ __forceinline__ void lsolve_tab(const TabRef lo, const TabRef H, int levels,
                                            int lane, V (&x)[NC][M]) {
-  RowStream<V, P, M> L;
+  RowStream<V, P * P, 1> hk[PRE ? 6 : 1];
+  if constexpr (PRE) {
 #pragma unroll
-  for (int t = 1; t < M; ++t) {
-    L.up(lo, t, 1);
+    for (int k = 0; k < 6; ++k) {
+      TabRef Hk = H;
+      Hk.sbias += k * P * P * WAVE * (int)sizeof(V);
+      if (k < levels) hk[k].up(Hk, 0);
+    }
+  }
+  RowStream<V, P, M> L;
+  constexpr int T0 = KEEP ? 0 : 1;  // row 0 has no row above it in the chunk
+#pragma unroll
+  for (int t = T0; t < M; ++t) {
+    L.up(lo, t, T0);
 #pragma unroll
     for (int i = 1; i <= P; ++i) {
       if (t - i < 0) continue;
@@ -421,17 +466,19 @@ __device__ __forceinline__ void lsolve_tab(const TabRef lo, const TabRef H, int 
   for (int k = 0; k < 6; ++k) {
     if (k < levels) {
       const int d = 1 << k;
-      // the level's composed map is loaded before the shuffles and outside
-      // the lane test, so its loads are in flight together
-      TabRef Hk = relaunder_after(H, c[0][0]);
-      Hk.sbias += k * P * P * WAVE * (int)sizeof(V);
-      RowStream<V, P * P, 1> h;
-      h.up(Hk, 0);
+      // without PRE the level's composed map is loaded before the shuffles
+      // and outside the lane test, so its loads are in flight together
+      auto& h = hk[PRE ? k : 0];
+      if constexpr (!PRE) {
+        TabRef Hk = relaunder_after(H, c[0][0]);
+        Hk.sbias += k * P * P * WAVE * (int)sizeof(V);
+        h.up(Hk, 0);
+      }
       V cp[NC][P];
 #pragma unroll
       for (int n = 0; n < NC; ++n)
 #pragma unroll
-        for (int q = 0; q < P; ++q) cp[n][q] = __shfl_up(c[n][q], d);
+        for (int q = 0; q < P; ++q) cp[n][q] = wave_up(c[n][q], d);
       if (lane >= d) {
 #pragma unroll
         for (int q = 0; q < P; ++q)
@@ -448,20 +495,20 @@ __device__ __forceinline__ void lsolve_tab(const TabRef lo, const TabRef H, int 
   for (int n = 0; n < NC; ++n)
 #pragma unroll
     for (int q = 0; q < P; ++q) {
-      const V v = __shfl_up(c[n][q], 1);
-      s[n][q] = lane == 0 ? V(0) : v;
+      s[n][q] = wave_up(c[n][q], 1);
     }
-  const TabRef lo2 = relaunder(lo);
   RowStream<V, P, M> L2;
+  TabRef lo2 = lo;
+  if constexpr (!KEEP) lo2 = relaunder(lo);
   V dl[NC][M];
 #pragma unroll
   for (int t = 0; t < M; ++t) {
-    L2.up(lo2, t);
+    if constexpr (!KEEP) L2.up(lo2, t);
 #pragma unroll
     for (int n = 0; n < NC; ++n) dl[n][t] = V(0);
 #pragma unroll
     for (int i = 1; i <= P; ++i) {
-      const V l = L2(t, i - 1);
+      const V l = KEEP ? L(t, i - 1) : L2(t, i - 1);
 #pragma unroll
       for (int n = 0; n < NC; ++n) {
         const V pv = (t - i >= 0) ? dl[n][t - i] : s[n][i - t - 1];
@@ -473,9 +520,18 @@ __device__ __forceinline__ void lsolve_tab(const TabRef lo, const TabRef H, int 
   }
 }
 
-template <int M, int P, int NC, typename V>
+template <int M, int P, int NC, bool KEEP, bool PRE, typename V>
 __device__ __forceinline__ void usolve_tab(const TabRef up, const TabRef H, int levels,
                                            int lane, V (&x)[NC][M]) {
+  RowStream<V, P * P, 1> hk[PRE ? 6 : 1];
+  if constexpr (PRE) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      TabRef Hk = H;
+      Hk.sbias += k * P * P * WAVE * (int)sizeof(V);
+      if (k < levels) hk[k].up(Hk, 0);
+    }
+  }
   RowStream<V, P + 1, M> U;
 #pragma unroll
   for (int t = M - 1; t >= 0; --t) {
@@ -501,15 +557,17 @@ __device__ __forceinline__ void usolve_tab(const TabRef up, const TabRef H, int 
   for (int k = 0; k < 6; ++k) {
     if (k < levels) {
       const int d = 1 << k;
-      TabRef Hk = relaunder_after(H, c[0][0]);
-      Hk.sbias += k * P * P * WAVE * (int)sizeof(V);
-      RowStream<V, P * P, 1> h;
-      h.up(Hk, 0);
+      auto& h = hk[PRE ? k : 0];
+      if constexpr (!PRE) {
+        TabRef Hk = relaunder_after(H, c[0][0]);
+        Hk.sbias += k * P * P * WAVE * (int)sizeof(V);
+        h.up(Hk, 0);
+      }
       V cp[NC][P];
 #pragma unroll
       for (int n = 0; n < NC; ++n)
 #pragma unroll
-        for (int q = 0; q < P; ++q) cp[n][q] = __shfl_down(c[n][q], d);
+        for (int q = 0; q < P; ++q) cp[n][q] = wave_down(c[n][q], d);
       if (lane + d < WAVE) {
 #pragma unroll
         for (int q = 0; q < P; ++q)
@@ -526,27 +584,27 @@ __device__ __forceinline__ void usolve_tab(const TabRef up, const TabRef H, int 
   for (int n = 0; n < NC; ++n)
 #pragma unroll
     for (int q = 0; q < P; ++q) {
-      const V v = __shfl_down(c[n][q], 1);
-      s[n][q] = lane == WAVE - 1 ? V(0) : v;
+      s[n][q] = wave_down(c[n][q], 1);
     }
-  const TabRef up2 = relaunder(up);
   RowStream<V, P + 1, M> U2;
+  TabRef up2 = up;
+  if constexpr (!KEEP) up2 = relaunder(up);
   V dl[NC][M];
 #pragma unroll
   for (int t = M - 1; t >= 0; --t) {
-    U2.down(up2, t);
+    if constexpr (!KEEP) U2.down(up2, t);
 #pragma unroll
     for (int n = 0; n < NC; ++n) dl[n][t] = V(0);
 #pragma unroll
     for (int d = 1; d <= P; ++d) {
-      const V u = U2(t, d);
+      const V u = KEEP ? U(t, d) : U2(t, d);
 #pragma unroll
       for (int n = 0; n < NC; ++n) {
         const V pv = (t + d < M) ? dl[n][t + d] : s[n][t + d - M];
         dl[n][t] -= u * pv;
       }
     }
-    const V iv = U2(t, 0);
+    const V iv = KEEP ? U(t, 0) : U2(t, 0);
 #pragma unroll
     for (int n = 0; n < NC; ++n) {
       dl[n][t] *= iv;
@@ -566,10 +624,8 @@ __device__ __forceinline__ void bmatvec(const TabRef B, int lane, const V (&u)[N
   for (int n = 0; n < NC; ++n)
 #pragma unroll
     for (int q = 0; q < P; ++q) {
-      const V a = __shfl_up(u[n][M - P + q], 1);
-      const V b = __shfl_down(u[n][q], 1);
-      hl[n][q] = lane == 0 ? V(0) : a;
-      hr[n][q] = lane == WAVE - 1 ? V(0) : b;
+      hl[n][q] = wave_up(u[n][M - P + q], 1);
+      hr[n][q] = wave_down(u[n][q], 1);
     }
   RowStream<V, 2 * P + 1, M> bc;
   if constexpr (ROWS) bc.up(B, 0);
@@ -615,7 +671,7 @@ __device__ __forceinline__ double col_value(const double (&x)[M], int row) {
 // streams of M rows of ytab_width entries a lane; the scan compositions of
 // the fixed factors are 6 streams (levels) of one P x P map a lane.
 enum YTabId {
-  YT_B1, YT_A1, YT_U1, YT_LO1, YT_FMAP,  // d/deta: B1, A1, LU of A1 (U: inv, up), fmap
+  YT_A1, YT_U1, YT_LO1, YT_FMAP,         // d/deta: A1, LU of A1 (U: inv, up), fmap
   YT_B2, YT_A2, YT_U2, YT_LO2,           // d2/dy2: B2, A2, LU of A2
   YT_UI, YT_LOI,                         // integration: LU of B1
   YT_WBD,                                // boundary d/dy functionals
@@ -625,7 +681,7 @@ enum YTabId {
 };
 __host__ __device__ constexpr int ytab_width(int id) {
   // entries per row of the per-row tables; P of the scan tables
-  return id == YT_B1 || id == YT_A1 ? 7
+  return id == YT_A1 ? 7
        : id == YT_B2 || id == YT_A2 ? 5
        : id == YT_U1 || id == YT_UI ? 4
        : id == YT_LO1 || id == YT_LOI || id == YT_U2 ? 3
@@ -633,7 +689,7 @@ __host__ __device__ constexpr int ytab_width(int id) {
        : id == YT_HL1 || id == YT_HU1 || id == YT_HLI || id == YT_HUI ? 3
        : id == YT_HL2 || id == YT_HU2 ? 2 : 1;
 }
-// element offset of table `id`; ytab_offset(YT_COUNT, M) is the total size
+// element offset of table `id`; the rows of B1 follow the last
 __host__ __device__ constexpr int ytab_offset(int id, int M) {
   int off = 0;
   for (int q = 0; q < id; ++q) {
@@ -642,6 +698,11 @@ __host__ __device__ constexpr int ytab_offset(int id, int M) {
   }
   return off;
 }
+// B1 is the same in every row but the first and last three (the grid of eta
+// is uniform): those six rows and the inner one, 7 entries each, padded to
+// whole vectors
+constexpr int B1_ROWS = 7, B1_SIZE = 52;
+__host__ __device__ constexpr int ytab_size(int M) { return ytab_offset(YT_COUNT, M) + B1_SIZE; }
 
 // Device tables of one y grid: one allocation, lane-major streams at the
 // offsets ytab_offset(id, M), so that every table access goes through one
@@ -662,15 +723,70 @@ __device__ __forceinline__ TabRef ytab(const YTab& T, int id, int lane) {
   return TabRef{make_rsrc(base, 0x7fffffff), lane * 16, ytab_offset(id, M) * (int)sizeof(V)};
 }
 
+// y = B1 u with the rows of B1 in scalar registers: no table load (32 of the
+// first derivative's 151 at M = 9).  Sums in the order of bmatvec.
+template <int M, int NC, typename V>
+__device__ __forceinline__ void b1_matvec(const YTab& T, int lane, const V (&u)[NC][M],
+                                          V (&y)[NC][M]) {
+  static_assert(M >= 3, "the edge rows span at most two lanes");
+  typedef const __attribute__((address_space(4))) V* crow;
+  const void* base = T.base;
+  if constexpr (sizeof(V) == 4) base = T.base32;
+  // opaque: the rows are read again in each operator, not kept through all
+  const V* rows = (const V*)base + ytab_offset(YT_COUNT, M);
+  asm volatile("" : "+s"(rows));
+  const crow E = (crow)rows;
+  V hl[NC][3], hr[NC][3];
+#pragma unroll
+  for (int n = 0; n < NC; ++n)
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      hl[n][q] = wave_up(u[n][M - 3 + q], 1);
+      hr[n][q] = wave_down(u[n][q], 1);
+    }
+  auto val = [&](int n, int col) __attribute__((always_inline)) {
+    return col < 0 ? hl[n][col + 3] : (col >= M ? hr[n][col - M] : u[n][col]);
+  };
+  auto edge = [&](int t, const crow c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int n = 0; n < NC; ++n) {
+      V acc = V(0);
+#pragma unroll
+      for (int d = 0; d < 7; ++d) acc += c[d] * val(n, t - 3 + d);
+      y[n][t] = acc;
+    }
+  };
+  // the last three rows: entry tb, tb + 1, tb + 2 of lane lb, running on into
+  // the next lane
+  const int my = T.my, lb = (my - 3) / M, tb = (my - 3) - lb * M;
+  V c[7];
+#pragma unroll
+  for (int d = 0; d < 7; ++d) c[d] = E[6 * 7 + d];
+#pragma unroll
+  for (int t = 0; t < M; ++t) {
+#pragma unroll
+    for (int n = 0; n < NC; ++n) {
+      V acc = V(0);
+#pragma unroll
+      for (int d = 0; d < 7; ++d)
+        if (d != 3) acc += c[d] * val(n, t - 3 + d);  // no diagonal inside
+      y[n][t] = lane * M + t < my ? acc : V(0);
+    }
+    if (t < 3 && lane == 0) edge(t, E + t * 7);
+    const int q = t - tb + (t < tb ? M : 0);
+    if (q < 3 && lane == lb + (t < tb ? 1 : 0)) edge(t, E + (3 + q) * 7);
+  }
+}
+
 // first derivative du = fmap * A1^{-1} B1 u   (deryr2, cfdiff.f:518-601)
-template <int M, int NC, typename V, bool ROWS = true>
+template <int M, int NC, typename V, bool KEEP = true, bool PRE = false>
 __device__ __forceinline__ void op_dy1(const YTab& T, int lane, const V (&u)[NC][M],
                                        V (&du)[NC][M], bool apply_fmap = true) {
-  bmatvec<M, 3, NC, V, ROWS>(ytab<M, V>(T, YT_B1, lane), lane, u, du);
+  b1_matvec<M, NC, V>(T, lane, u, du);
   op_fence();
-  lsolve_tab<M, 3, NC>(ytab<M, V>(T, YT_LO1, lane), ytab<M, V>(T, YT_HL1, lane), T.kL1, lane, du);
+  lsolve_tab<M, 3, NC, KEEP, PRE>(ytab<M, V>(T, YT_LO1, lane), ytab<M, V>(T, YT_HL1, lane), T.kL1, lane, du);
   op_fence();
-  usolve_tab<M, 3, NC>(ytab<M, V>(T, YT_U1, lane), ytab<M, V>(T, YT_HU1, lane), T.kU1, lane, du);
+  usolve_tab<M, 3, NC, KEEP, PRE>(ytab<M, V>(T, YT_U1, lane), ytab<M, V>(T, YT_HU1, lane), T.kU1, lane, du);
   op_fence();
   if (apply_fmap) {
     RowStream<V, 1, M> fm;
@@ -686,14 +802,14 @@ __device__ __forceinline__ void op_dy1(const YTab& T, int lane, const V (&u)[NC]
 }
 
 // second derivative d2u = A2^{-1} B2 u   (deryyr2, cfdiff.f:735-797)
-template <int M, int NC, typename V, bool ROWS = true>
+template <int M, int NC, typename V, bool ROWS = true, bool KEEP = true, bool PRE = false>
 __device__ __forceinline__ void op_dy2(const YTab& T, int lane, const V (&u)[NC][M],
                                        V (&d2u)[NC][M]) {
   bmatvec<M, 2, NC, V, ROWS>(ytab<M, V>(T, YT_B2, lane), lane, u, d2u);
   op_fence();
-  lsolve_tab<M, 2, NC>(ytab<M, V>(T, YT_LO2, lane), ytab<M, V>(T, YT_HL2, lane), T.kL2, lane, d2u);
+  lsolve_tab<M, 2, NC, KEEP, PRE>(ytab<M, V>(T, YT_LO2, lane), ytab<M, V>(T, YT_HL2, lane), T.kL2, lane, d2u);
   op_fence();
-  usolve_tab<M, 2, NC>(ytab<M, V>(T, YT_U2, lane), ytab<M, V>(T, YT_HU2, lane), T.kU2, lane, d2u);
+  usolve_tab<M, 2, NC, KEEP, PRE>(ytab<M, V>(T, YT_U2, lane), ytab<M, V>(T, YT_HU2, lane), T.kU2, lane, d2u);
   op_fence();
 }
 

@@ -316,8 +316,8 @@ __device__ __forceinline__ void op_inty(const YTab& T, int lane, double (&x)[1][
 #pragma unroll
   for (int t = 0; t < M; ++t)
     if (r0 + t == T.my - 1) x[0][t] = 0.0;  // gauge row x(my) = 0
-  lsolve_tab<M, 3, 1>(ytab<M>(T, YT_LOI, lane), ytab<M>(T, YT_HLI, lane), T.kLi, lane, x);
-  usolve_tab<M, 3, 1>(ytab<M>(T, YT_UI, lane), ytab<M>(T, YT_HUI, lane), T.kUi, lane, x);
+  lsolve_tab<M, 3, 1, true, M <= 3>(ytab<M>(T, YT_LOI, lane), ytab<M>(T, YT_HLI, lane), T.kLi, lane, x);
+  usolve_tab<M, 3, 1, true, M <= 3>(ytab<M>(T, YT_UI, lane), ytab<M>(T, YT_HUI, lane), T.kUi, lane, x);
   const double v0 = col_value<M>(x[0], 0);
 #pragma unroll
   for (int t = 0; t < M; ++t) x[0][t] -= v0;
@@ -527,12 +527,12 @@ __global__ __launch_bounds__(256, 3) void k_phaseC32_batch(const PhaseArgs* __re
 // from the class table (the second Dirichlet solve of solvepsi, laps.f:
 // 700-726, by linearity).  The class with kx = kz = 0 is the 00 mode alone.
 template <int M, typename TS>
-__global__ __launch_bounds__(256) void k_phaseC2(PhaseArgs a) {
+__global__ __launch_bounds__(256, M <= 9 ? 2 : 1) void k_phaseC2(PhaseArgs a) {
   const int bx = blockIdx.x;
 #include "loma_phaseC2_body.inc"
 }
 template <int M, typename TS>
-__global__ __launch_bounds__(256) void k_phaseC2_batch(const PhaseArgs* __restrict__ args,
+__global__ __launch_bounds__(256, M <= 9 ? 2 : 1) void k_phaseC2_batch(const PhaseArgs* __restrict__ args,
     const int* __restrict__ first, int nrun) {
   const int r = wave_uniform(batch_run(first, nrun, blockIdx.x));
   const PhaseArgs& a = args[r];
