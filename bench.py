@@ -40,8 +40,8 @@ MEASURED_TRAFFIC = {
 }
 
 
-_TRAFFIC_KEYS = {"k_phaseA": "phaseA", "k_zfft_inv": "zfft_inv", "k_xline": "xline",
-                 "k_zfft_fwd": "zfft_fwd", "k_phaseC": "phaseC", "k_phaseC32": "phaseC",
+_TRAFFIC_KEYS = {"k_phaseA": "phaseA", "k_zfft_inv": "zfft_inv", "k_xrow": "xline",
+                 "k_xline": "xline", "k_zfft_fwd": "zfft_fwd", "k_phaseC": "phaseC", "k_phaseC32": "phaseC",
                  "k_phaseC2": "phaseC2"}
 
 
@@ -126,11 +126,12 @@ def algorithmic_bytes(run, with_z: bool):
     """Compulsory HBM bytes per launch of each kernel class (one substep)
     and per RK3 step: one read of every field a kernel consumes and one write
     of every field it produces (S, W, P sized; es bytes per complex transform
-    entry), nothing else."""
+    entry), nothing else.  The fields are those of foup2 (8 in, 11 out); a
+    step transforms one less each way, which the measured traffic shows."""
     S, W, P = run.S, run.W, run.P
     es = 8 if run.precision == 1 else 16
     z = 1 if with_z else 0
-    nin, nout = (11, 11) if with_z else (7, 10)
+    nin, nout = (12, 12) if with_z else (8, 11)
     k = {
         # reads phi, ten13, vor, ten12, psi, T (+Z); writes phi, vor; writes
         # the transform inputs
