@@ -1155,12 +1155,16 @@ static int autotune_tiles(loma_run* r) {
   }
   r->J = bestJ;
   best = 1e30f;
-  for (int L = L0; L >= 2 && L >= L0 / 4; L /= 2) {
-    r->L = L;
-    int e = time_launch(r, 1, &ms);
-    if (e) return e;
-    if (ms < best) { best = ms; bestL = L; }
-  }
+  // The row kernel's tile stays: at another one its lengths run k_xline, whose
+  // passes round differently, and a timing would choose a run's result (mixed
+  // runs: at FP32 level).
+  if (!xrow_serves(r->fp32, fft_args(r, 1, 0)))
+    for (int L = L0; L >= 2 && L >= L0 / 4; L /= 2) {
+      r->L = L;
+      int e = time_launch(r, 1, &ms);
+      if (e) return e;
+      if (ms < best) { best = ms; bestL = L; }
+    }
   r->L = bestL;
   std::lock_guard<std::mutex> lk(g_tile_mu);
   g_tiles.push_back({key, {bestJ, bestL}});
