@@ -674,12 +674,18 @@ __device__ __forceinline__ void xl_pack_from(const FftArgs& a, const XlIn<T2, XR
       const int it = threadIdx.x + r * XL_THREADS;
       if (it < np * pairs) {
         const int ii = it >> lp, p = it & (pairs - 1);
-        T2 ca = v[f].a[r], cb = v[f].b[r];
+        const T2 ca = v[f].a[r], cb = v[f].b[r];
         const int rb = (f * pairs + p) * RS;
-        if (f == dx) {                // this field times ikx
-          const T kx = (T)(a.rc.alp * ii);
-          ca = T2{-ca.y * kx, ca.x * kx};
-          cb = T2{-cb.y * kx, cb.x * kx};
+        if (f == dx) {                // ikx times this field, rounded once (XRow::pack_dx)
+          const double kx = a.rc.alp * ii;
+          const double ax = -kx * ca.y, ay = kx * ca.x, bx = -kx * cb.y, by = kx * cb.x;
+          if (ii == 0) {
+            A[lds_i<XP>(rb)] = T2{(T)ax, (T)bx};
+          } else {
+            A[lds_i<XP>(rb + ii)] = T2{(T)(ax - by), (T)(ay + bx)};
+            A[lds_i<XP>(rb + N - ii)] = T2{(T)(ax + by), (T)(-ay + bx)};
+          }
+          continue;
         }
         if (ii == 0) {
           // the imaginary part of the kx=0 coefficient is ignored (rft, rftsingle.f:87-91)
@@ -902,8 +908,9 @@ struct XRow {
       v.b[r] = T2{q[2], q[3]};
     }
   }
-  // the coefficients times ikx
+  // the coefficients times ikx (FP64; FP32 rows take pack_dx)
   __device__ static __forceinline__ void ikx(XlIn<T2, XR>& v, int tg, double alp) {
+    static_assert(sizeof(T) == 8, "kx and the products are FP64");
 #pragma unroll
     for (int r = 0; r < XR; ++r) {
       const T kx = (T)(alp * ((tg + r * GT) / P));
@@ -911,11 +918,9 @@ struct XRow {
       v.b[r] = T2{-v.b[r].y * kx, v.b[r].x * kx};
     }
   }
-  // two real lines to one complex row; the imaginary part of the kx = 0
-  // coefficient is ignored (rft, rftsingle.f:87-91).  left: lines of the tile
-  // inside the grid (the others read as zero)
-  __device__ static __forceinline__ void pack(XlIn<T2, XR> v, T2* A, int tg, const Items& t,
-                                              int left) {
+  // left: lines of the tile inside the grid (the others read as zero); the
+  // imaginary part of the kx = 0 coefficient is ignored (rft, rftsingle.f:87-91)
+  __device__ static __forceinline__ void mask(XlIn<T2, XR>& v, int tg, int left) {
     if (left < 2 * P) {
 #pragma unroll
       for (int r = 0; r < XR; ++r) {
@@ -928,11 +933,31 @@ struct XRow {
     }
     v.a[0].y = tg < P ? (T)0 : v.a[0].y;
     v.b[0].y = tg < P ? (T)0 : v.b[0].y;
+  }
+  // two real lines to one complex row
+  __device__ static __forceinline__ void pack(XlIn<T2, XR> v, T2* A, int tg, const Items& t,
+                                              int left) {
+    mask(v, tg, left);
 #pragma unroll
     for (int r = 0; r < XR; ++r) {
       const T2 ca = v.a[r], cb = v.b[r];
       A[t.lo[r]] = T2{ca.x - cb.y, ca.y + cb.x};      // X_a + i X_b
       A[t.hi[r]] = T2{ca.x + cb.y, -ca.y + cb.x};     // conj(X_a) + i conj(X_b)
+    }
+  }
+  // the rows of d/dx: X = ikx times the coefficients, formed and summed in FP64
+  // and rounded once (kx and the products rounded to FP32 on their own put two
+  // more roundings on dT/dx)
+  __device__ static __forceinline__ void pack_dx(XlIn<T2, XR> v, T2* A, int tg, const Items& t,
+                                                 int left, double alp) {
+    mask(v, tg, left);
+#pragma unroll
+    for (int r = 0; r < XR; ++r) {
+      const double kx = alp * ((tg + r * GT) / P);
+      const double ax = -kx * v.a[r].y, ay = kx * v.a[r].x;
+      const double bx = -kx * v.b[r].y, by = kx * v.b[r].x;
+      A[t.lo[r]] = T2{(T)(ax - by), (T)(ay + bx)};
+      A[t.hi[r]] = T2{(T)(ax + by), (T)(-ay + bx)};
     }
   }
   // entry jl + c of a packed row (c a multiple of 8); NP .. N-NP are zero
