@@ -550,8 +550,11 @@ __global__ __launch_bounds__(256, M <= 9 ? 2 : 1) void k_phaseC2_batch(const Pha
 //   pass 2: rho u_i = rho scale_c c_i; psi from lap psi = div(rho u)
 //   (Lapvdvhom, main.f:452-463); Omega_y = ikz rho u - ikx rho w;
 //   phi = (D2 - k^2)(rho v - d psi/dy); T and Z in the 00 mode only.
+// Two waves a SIMD up to M = 5: there it is ten registers past, and a
+// loma_seed of 200x257x160 takes 475 us with two waves (ten registers spilled)
+// and 585 with one.
 template <int M>
-__global__ __launch_bounds__(256) void k_ic(IcArgs a) {
+__global__ __launch_bounds__(256, M <= 5 ? 2 : 1) void k_ic(IcArgs a) {
   LOMA_STAGE(M);
   const RunConst& rc = a.rc;
   const int nmodes = rc.nplanes * rc.mz;
