@@ -707,26 +707,46 @@ static int get_fields(loma_run* r, int nf, const double2* const* src, void* cons
   const size_t n = 2 * S;
   const int nslot = (int)std::min<size_t>(HSTAGE_SLOTS, std::max<size_t>(1, n / (64 << 10)));
   const size_t len = ((n + nslot - 1) / nslot + 511) / 512 * 512;  // numbers per slot
-  for (int q = 0; q < nslot; ++q)
-    if (!r->hev[q]) HIPCHK(hipEventCreateWithFlags(&r->hev[q], hipEventDisableTiming));
   int f[4], m = 0;
   for (int q = 0; q < nf; ++q)
     if (dst[q]) f[m++] = q;
   if (!m) return LOMA_OK;
   auto count = [&](int q) { return q * len < n ? std::min(len, n - q * len) : 0; };
-  auto fill = [&](int k, int q) -> hipError_t {  // slot q of field f[k]
+  auto copy = [&](int k, int q) -> hipError_t {  // slot q of field f[k] into the staging
     const double* p = (const double*)src[f[k]] + q * len;
-    if (!count(q)) return hipSuccess;
-    hipError_t e;
-    if (fp64) {
-      e = hipMemcpyAsync(r->hstage + q * len, p, count(q) * sizeof(double), hipMemcpyDeviceToHost,
-                         r->stream);
-    } else {
-      e = (hipError_t)launch_narrow(p, (float*)(r->hstage + q * len), count(q), r->stream);
-    }
-    return e != hipSuccess ? e : hipEventRecord(r->hev[q], r->stream);
+    if (fp64)
+      return hipMemcpyAsync(r->hstage + q * len, p, count(q) * sizeof(double),
+                            hipMemcpyDeviceToHost, r->stream);
+    return (hipError_t)launch_narrow(p, (float*)(r->hstage + q * len), count(q), r->stream);
   };
   const size_t el = fp64 ? sizeof(double) : sizeof(float);
+  if (nslot == 1) {
+    // Nothing to overlap: a wait for the stream costs less than an event a
+    // field (48x97x36: 187 us an image, 247 with events).  The smallest FP32
+    // fields are rounded here: a copy and a loop cost less than the kernel
+    // (16x33x12: 69 against 81 us; equal at some 20,000 numbers).
+    const bool host_round = !fp64 && n <= (16 << 10);
+    for (int k = 0; k < m; ++k) {
+      if (host_round)
+        HIPCHK(hipMemcpyAsync(r->hstage, src[f[k]], n * sizeof(double), hipMemcpyDeviceToHost,
+                              r->stream));
+      else
+        HIPCHK(copy(k, 0));
+      HIPCHK(hipStreamSynchronize(r->stream));
+      if (host_round)
+        for (size_t i = 0; i < n; ++i) ((float*)dst[f[k]])[i] = (float)r->hstage[i];
+      else
+        std::memcpy(dst[f[k]], r->hstage, n * el);
+    }
+    return LOMA_OK;
+  }
+  for (int q = 0; q < nslot; ++q)
+    if (!r->hev[q]) HIPCHK(hipEventCreateWithFlags(&r->hev[q], hipEventDisableTiming));
+  auto fill = [&](int k, int q) -> hipError_t {
+    if (!count(q)) return hipSuccess;
+    const hipError_t e = copy(k, q);
+    return e != hipSuccess ? e : hipEventRecord(r->hev[q], r->stream);
+  };
   auto drain = [&](int t, int nt) -> hipError_t {  // slots t, t + nt, ...
     for (int k = 0; k < m; ++k)
       for (int q = t; q < nslot; q += nt) {
