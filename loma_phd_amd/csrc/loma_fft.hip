@@ -1371,11 +1371,13 @@ int launch_fourz(const FftPlan& pl, const double2* tw, double2* c, int nrows, in
     LOMA_FOURZ_ROW(256) LOMA_FOURZ_ROW(384) LOMA_FOURZ_ROW(512)
 #undef LOMA_FOURZ_ROW
     default: {
-      // a butterfly's radix is at most 8: 2048 entries keep 256 threads busy
-      // (both buffers 72 KiB); longer rows go one to a workgroup.  Few rows are
-      // spread over the chip first, four workgroups to a CU: 734 rows of 216 take
-      // 20 us nine to a workgroup and 17 us one to a workgroup
-      const int per = std::max(1, std::min(2048 / pl.n, nrows / 1024));
+      // 1024 entries a workgroup (both buffers 32 KiB: five workgroups a CU hide
+      // each other's barriers); longer rows go one to a workgroup.  2048 entries
+      // leave two a CU: 50,001 rows of 480 take 341 us so, 224 with 1024 and 299
+      // with one row a workgroup; 5,003 rows of 1000 take 66, 51 and 53.  Few rows
+      // are spread over the chip first, four workgroups to a CU: 734 rows of 216
+      // take 20 us nine to a workgroup and 17 us one to a workgroup
+      const int per = std::max(1, std::min(1024 / pl.n, nrows / 1024));
       hipLaunchKernelGGL(k_fourz, dim3((nrows + per - 1) / per), dim3(256),
                          (size_t)2 * lds_entries(pl.n * per) * 16, st, pl, tw, c, nrows, iopt, per);
     }
