@@ -156,11 +156,32 @@ __global__ __launch_bounds__(64) void k_helm_factor(const double* __restrict__ d
   }
   __syncthreads();
   const int s = blockIdx.x * 64 + threadIdx.x;
-  if (s >= nsys) return;
-  const double sh = shifts[s] + shift;
   const int stride = 5 * WAVE * M * 8;  // bytes of a system's table
   const auto out = make_rsrc(lu + (size_t)blockIdx.x * 64 * (5 * WAVE * M), 0x7fffffff);
   const int vo = threadIdx.x * stride;
+  const int ubase = 2 * WAVE * M * 8;
+  // The rows past my-1 are zero.  A batch of a few systems clears them with the
+  // lanes along the rows, system by system (0.24 us for 64 rows of one), others
+  // with each lane its own system's behind the chain (0.09 us a row, whatever
+  // the systems): one visc of 17 rows, 175 of 192 to clear, 58 against 89 us.
+  const int pad = WAVE * M - my, nb = min(64, nsys - (int)blockIdx.x * 64);
+  const bool together = 4 * nb * ((pad + 63) / 64) < pad;
+  if (together)
+    for (int q = 0; q < nb; ++q)
+      for (int r = my + (int)threadIdx.x; r < WAVE * M; r += 64) {
+        typedef unsigned u2v __attribute__((ext_vector_type(2)));
+        const int l = r / M, t = r - l * M, sys = q * stride;
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+          __builtin_amdgcn_raw_buffer_store_b64(
+              u2v{0, 0}, out, sys + ubase + stream_index(3 * M, 3 * t + e, l, 2) * 8, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          __builtin_amdgcn_raw_buffer_store_b64(
+              u2v{0, 0}, out, sys + stream_index(2 * M, 2 * t + e, l, 2) * 8, 0, 0);
+      }
+  if (s >= nsys) return;
+  const double sh = shifts[s] + shift;
   auto put = [&](int so, double v) {
     typedef unsigned u2v __attribute__((ext_vector_type(2)));
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2v, v), out, vo, so, 0);
@@ -176,7 +197,7 @@ __global__ __launch_bounds__(64) void k_helm_factor(const double* __restrict__ d
   };
   int l = 0, t = 0, ln = 0, tn = 1;  // lane and slot of rows k and k+1 (M >= 3)
   double l2 = 0.0;                   // row k-1's multiplier into row k+1
-  const int ubase = 2 * WAVE * M * 8, utail = ubase + (3 * M - 1) * (WAVE * 8);
+  const int utail = ubase + (3 * M - 1) * (WAVE * 8);
   const int tlast = (M & 1) ? M - 1 : -1;  // slot whose up2 lies behind the vectors
   auto store_row = [&](double iv, double u1, double u2, double m1, double m2) {
     // entries 3t .. 3t+2 of lane l's U stream, two to a 16-byte vector
@@ -257,7 +278,8 @@ __global__ __launch_bounds__(64) void k_helm_factor(const double* __restrict__ d
 #pragma unroll
     for (int d = 0; d < 5; ++d) { w0[d] = w1[d]; w1[d] = w2[d]; w2[d] = w3[d]; }
   }
-  for (; k < WAVE * M; ++k) store_row(0.0, 0.0, 0.0, 0.0, 0.0);
+  if (!together)
+    for (; k < WAVE * M; ++k) store_row(0.0, 0.0, 0.0, 0.0, 0.0);
 }
 
 int launch_helm_factor(const double* dt21, const double* dt22, int my, int M,
