@@ -118,7 +118,7 @@ struct loma_run {
   int snap_istep = -1;
   // statistics window (loma_stats_*): device accumulators, the spectra rows
   // and the host-side switch and counter; allocated by loma_stats_config
-  double *st_acc = nullptr, *st_spe = nullptr, *st_part = nullptr, *st_rho = nullptr,
+  double *st_acc = nullptr, *st_spe = nullptr, *st_part = nullptr, *st_lines = nullptr,
          *st_last = nullptr;
   int* st_jsp = nullptr;
   // workspace of the batched solves (solve_ws)
@@ -333,7 +333,7 @@ int loma_free(loma_run* r) {
   if (r->snap) hipFree(r->snap);
   if (r->ws) hipFree(r->ws);
   if (r->ws_ev) hipEventDestroy(r->ws_ev);
-  for (void* p : {(void*)r->st_acc, (void*)r->st_spe, (void*)r->st_part, (void*)r->st_rho,
+  for (void* p : {(void*)r->st_acc, (void*)r->st_spe, (void*)r->st_part, (void*)r->st_lines,
                   (void*)r->st_last, (void*)r->st_jsp})
     if (p) hipFree(p);
   if (r->owns_stream && r->stream) hipStreamDestroy(r->stream);
@@ -1079,7 +1079,7 @@ static StatsArgs stats_args(loma_run* r) {
   a.acc = r->st_acc;
   a.spe = r->st_spe;
   a.part = r->st_part;
-  a.rho = r->st_rho;
+  a.lines = r->st_lines;
   a.last = r->st_last;
   return a;
 }
@@ -1092,8 +1092,7 @@ static int enqueue_substep(loma_run* r, int rkstep, int icfl) {
   PROF(KC_PHASEA, launch_phaseA(r->M, r->fp32, pa, st));
   if (stats) LCHK(launch_stats(r->M, r->fp32, 1, stats_args(r), st));
   FftArgs fa = fft_args(r, rkstep, (rkstep == 1 && icfl) ? 1 : 0);
-  fa.stat_rho = stats ? r->st_rho : nullptr;
-  fa.out_rvv = stats ? 1 : 0;
+  fa.stat_lines = stats ? r->st_lines : nullptr;
   fa.nfields = xf_inputs(fa);
   PROF(KC_ZINV, launch_zfft_inv(r->fp32, fa, st));
   PROF(KC_XLINE, launch_xline(r->fp32, fa, st));
@@ -1851,16 +1850,16 @@ int loma_stats_config(loma_run* r, int nspec, const int* jspecy) {
   std::lock_guard<std::recursive_mutex> lk(g_setup_mu);
   if (r->stream) HIPCHK(hipStreamSynchronize(r->stream));
   for (void** p : {(void**)&r->st_acc, (void**)&r->st_spe, (void**)&r->st_part,
-                   (void**)&r->st_rho, (void**)&r->st_last, (void**)&r->st_jsp})
+                   (void**)&r->st_lines, (void**)&r->st_last, (void**)&r->st_jsp})
     if (*p) { hipFree(*p); *p = nullptr; }
   const int nsp = (int)rows.size();
   const size_t nacc = (size_t)STAT_NCOL * my;
   const size_t nspe = (size_t)r->nplanes * 12 * nsp * (r->nz + 1);
   const size_t npart = (size_t)r->nplanes * ((r->nz + STAT_KACH) / STAT_KACH) * STAT_NPART * my;
-  const size_t nrho = (size_t)r->mgalz * my;
+  const size_t nline = (size_t)4 * r->mgalz * my;
   struct { void** p; size_t bytes; } al[] = {
       {(void**)&r->st_acc, nacc * 8}, {(void**)&r->st_spe, nspe * 8},
-      {(void**)&r->st_part, npart * 8}, {(void**)&r->st_rho, nrho * 8},
+      {(void**)&r->st_part, npart * 8}, {(void**)&r->st_lines, nline * 8},
       {(void**)&r->st_last, (size_t)9 * my * 8}, {(void**)&r->st_jsp, (size_t)nsp * 4}};
   for (auto& a : al) {
     if (hipMalloc(a.p, a.bytes) != hipSuccess) {

@@ -112,9 +112,9 @@ struct FftArgs {
   // CFL maxima of each x-line tile, [tile][4]: max |u|, max |v|/hy, max |w|,
   // max diffusive inverse dt (written by the substep that takes the CFL)
   double* cflp;
-  // per-line sums of 1/T over x, [mgalz][my] (statistics steps only; null
-  // otherwise)
-  double* stat_rho;
+  // sums over x of each line's 1/T and of ruu, rvv, rww less the product of
+  // their profiles, [4][mgalz][my] (statistics steps only; null otherwise)
+  double* stat_lines;
   int nfields;
   int rkstep;
   int do_cfl;
@@ -123,17 +123,16 @@ struct FftArgs {
   int L;                     // lines per x-line block
   // x lines: foup2's own fields (dT/dx comes in slot 4; outputs 3, 4, 5 are
   // ruu, rvv, rww).  Else the step's: dT/dx is ikx T, outputs 3 and 5 are
-  // ruu - rvv and rww - rvv, and rvv goes to slot 4 only with out_rvv
+  // ruu - rvv and rww - rvv
   int full;
-  int out_rvv;
   int xrow;                  // x lines by k_xrow (xrow_serves)
 };
 
 // The transform fields of a step.  Slot 4 stays empty both ways: dT/dx needs
 // no transform of its own in z (ikx commutes with it), and the step needs
-// rvv only in ruu - rvv and rww - rvv (loma_phaseC_body.inc).  Statistics
-// take the plane sums of ruu, rvv, rww and have rvv as well.  17 fields pass
-// the z transforms instead of 19 (22 instead of 24 with Z): at 512x513x256 a
+// rvv only in ruu - rvv and rww - rvv (loma_phaseC_body.inc; statistics take
+// the plane sums of ruu, rvv, rww from the lines).  17 fields pass the z
+// transforms instead of 19 (22 instead of 24 with Z): at 512x513x256 a
 // step takes 20.0 instead of 21.5 ms (FP64) and 12.2 instead of 12.9 ms
 // (mixed).  The differences are taken to rvv so that -rK rvv + kx^2 ruu +
 // kz^2 rww, the sum phi needs, is kx^2 (ruu - rvv) + kz^2 (rww - rvv): no
@@ -144,10 +143,10 @@ __host__ __device__ inline int xf_inputs(const FftArgs& a) {
 // the slot left out (12: none)
 __host__ __device__ inline int xf_skip_in(const FftArgs& a) { return a.full ? 12 : 4; }
 __host__ __device__ inline int xf_outputs(const FftArgs& a) {
-  return (a.with_z ? 12 : 11) - (a.full || a.out_rvv ? 0 : 1);
+  return (a.with_z ? 12 : 11) - (a.full ? 0 : 1);
 }
 __host__ __device__ inline int xf_skip_out(const FftArgs& a) {
-  return a.full || a.out_rvv ? 12 : 4;
+  return a.full ? 12 : 4;
 }
 
 // statistics window (addstats1/2 and the phys2 sums of cross.f): the
@@ -172,7 +171,7 @@ struct StatsArgs {
   double* acc;               // [STAT_NCOL][my]
   double* spe;               // [nplanes][12][nsp][nz+1]
   double* part;              // [STAT_NPART][my][nw], this step's sums per chunk
-  const double* rho;         // [mgalz][my] line sums of 1/T from the x lines
+  const double* lines;       // [4][mgalz][my] line sums from the x lines (FftArgs)
   double* last;              // [9][my] this step's plane-summed intensities (uner)
 };
 

@@ -104,8 +104,7 @@ __global__ __launch_bounds__(256) void k_stats_in(StatsArgs a) {
 // ikx w, o3 = ikx v - du/dy).  The twelve per-y sums of a mode go to LDS
 // (one column each, row t*64 + lane of the lane's own rows), the chunk's
 // totals to its partial.  The wavefront of plane 0, chunk 0 also adds the
-// 00 means and the phys2 sums of rho u_i u_j, which are the 00 mode of the
-// transformed products times mgalx*mgalz (cross.f:1586-1601).
+// 00 means and the phys2 sums of rho u_i u_j (cross.f:1586-1601).
 template <int M, typename TS>
 __global__ __launch_bounds__(64) void k_stats_out(StatsArgs a) {
   using T2 = typename std::conditional<sizeof(TS) == 4, float2, double2>::type;
@@ -242,28 +241,27 @@ __global__ __launch_bounds__(64) void k_stats_out(StatsArgs a) {
       if (r0 + t < my)
         a.part[((size_t)(1 + q) * my + r0 + t) * a.nw + wv] = sacc[q][t * WAVE + lane];
   if (wv == 0) {
-    // sum over the plane of rho u_i u_j = mgalx*mgalz times the 00 mode of
-    // the transformed product (slot -> column: 3 ruu, 6 ruv, 7 ruw, 4 rvv,
-    // 8 rvw, 5 rww; slots 3 and 5 hold ruu - rvv and rww - rvv)
+    // sum over the plane of rho u_i u_j: of ruv, ruw, rvw mgalx*mgalz times the
+    // 00 mode of the transformed product (slots 6, 7, 8); of ruu, rvv, rww that
+    // of their profiles (k_stats_reduce adds the lines' sums, in FP64 of each
+    // product by itself: the transforms carry differences of them, whose
+    // rounding is that of the largest)
     const double npts = (double)rc.mgalx * (double)rc.mgalz;
-    const int slot[6] = {3, 6, 7, 4, 8, 5};
+    constexpr int col[3] = {23, 24, 26}, dia[3] = {22, 25, 27};
 #pragma unroll 1
-    for (int q = 0; q < 6; ++q) {
+    for (int q = 0; q < 3; ++q) {
       double x[2][M];
       wave_sync();
-      load_col<M>((const T2*)a.spec[slot[q]], my, lane, st, x);
-      add_mean<M>(x, lane, my, true, a.mean_out + (size_t)slot[q] * my);
-      if (q == 0 || q == 5) {
-        double v[2][M];
-        wave_sync();
-        load_col<M>((const T2*)a.spec[4], my, lane, st, v);
-        add_mean<M>(v, lane, my, true, a.mean_out + (size_t)4 * my);
-#pragma unroll
-        for (int t = 0; t < M; ++t) x[0][t] += v[0][t];
-      }
+      load_col<M>((const T2*)a.spec[6 + q], my, lane, st, x);
+      add_mean<M>(x, lane, my, true, a.mean_out + (size_t)(6 + q) * my);
 #pragma unroll
       for (int t = 0; t < M; ++t)
-        if (r0 + t < my) a.acc[(size_t)(22 + q) * my + r0 + t] += npts * x[0][t];
+        if (r0 + t < my) {
+          const int r = r0 + t;
+          const double m = a.mean_in[(size_t)q * my + r];
+          a.acc[(size_t)col[q] * my + r] += npts * x[0][t];
+          a.acc[(size_t)dia[q] * my + r] += npts * (m * (m * a.mean_in[(size_t)7 * my + r]));
+        }
     }
   }
 }

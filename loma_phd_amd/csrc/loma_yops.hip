@@ -357,13 +357,15 @@ int launch_finish_batch(const FinishArgs* args, int nrun, hipStream_t st) {
 __global__ __launch_bounds__(64) void k_stats_reduce(StatsArgs a) {
   const int my = a.rc.my;
   const int j = blockIdx.x, q = blockIdx.y, lane = threadIdx.x;
-  constexpr int col[STAT_NPART + 1] = {20, 11, 12, 13, 14, 15, 16, 17, 18, 19, 29, 30, 21, 28};
+  constexpr int col[STAT_NPART + 4] = {20, 11, 12, 13, 14, 15, 16, 17, 18,
+                                       19, 29, 30, 21, 28, 22, 25, 27};
   double s = 0.0;
   if (q < STAT_NPART) {
     const double* p = a.part + ((size_t)q * my + j) * a.nw;
     for (int w = lane; w < a.nw; w += 64) s += p[w];
   } else {
-    for (int z = lane; z < a.rc.mgalz; z += 64) s += a.rho[(size_t)z * my + j];
+    const double* p = a.lines + (size_t)(q - STAT_NPART) * a.rc.mgalz * my;
+    for (int z = lane; z < a.rc.mgalz; z += 64) s += p[(size_t)z * my + j];
   }
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) s += __shfl_xor(s, d);
@@ -375,7 +377,7 @@ __global__ __launch_bounds__(64) void k_stats_reduce(StatsArgs a) {
 
 int launch_stats(int M, bool fp32, int which, const StatsArgs& a, hipStream_t st) {
   if (which == 3) {
-    hipLaunchKernelGGL(k_stats_reduce, dim3(a.rc.my, STAT_NPART + 1), dim3(64), 0, st, a);
+    hipLaunchKernelGGL(k_stats_reduce, dim3(a.rc.my, STAT_NPART + 4), dim3(64), 0, st, a);
     return (int)hipGetLastError();
   }
   LOMA_DISPATCH_M(M, launch_stats_m<MM>(fp32, which, a, st));
