@@ -203,6 +203,34 @@ __device__ __forceinline__ void twiddle_pow(T2* w, T2 p1, int s) {
 #pragma unroll
   for (int r = 1; r < R; ++r) w[r] = cmul(w[r], p[r]);
 }
+// The same with the third power p3 from the table too: no power is more than
+// two multiplications away from a table entry.  The recursion from p1 alone
+// makes most of a transform's error and grows with the radices of the later
+// passes (rms of 256 points in eps: passes 8, 8, 4 1.02 FP32 and 1.09 FP64;
+// 4, 8, 8 1.40 and 1.30, with p3 0.79 and 0.70).
+template <int R, typename T2>
+__device__ __forceinline__ void twiddle_pow3(T2* w, T2 p1, T2 p3, int s) {
+  if constexpr (R < 4) {
+    twiddle_pow<R>(w, p1, s);
+  } else {
+    T2 p[R];
+    p[1] = p1;
+    p[3] = p3;
+    if (s > 0) {
+      p[1].y = -p[1].y;
+      p[3].y = -p[3].y;
+    }
+    p[2] = cmul(p[1], p[1]);
+    if constexpr (R >= 5) p[4] = cmul(p[3], p[1]);
+    if constexpr (R >= 6) p[5] = cmul(p[3], p[2]);
+    if constexpr (R >= 8) {
+      p[6] = cmul(p[3], p[3]);
+      p[7] = cmul(p[4], p[3]);
+    }
+#pragma unroll
+    for (int r = 1; r < R; ++r) w[r] = cmul(w[r], p[r]);
+  }
+}
 template <int R, typename T2>
 __device__ __forceinline__ void twiddle(T2* w, const T2* __restrict__ tw, int jm, int tstep,
                                         int s) {
@@ -863,17 +891,25 @@ struct XRow {
   __device__ static __forceinline__ constexpr int li(int i) { return i + (i >> 3); }
   // position of entry jl + RL r (RL is a multiple of 8)
   __device__ static __forceinline__ int at(int jl, int r) { return li(jl) + RL / 8 * 9 * r; }
-  // first twiddles of the passes for lane jl
+  // Twiddles of lane jl, passes 0: first inverse, 1: second inverse, 2: first
+  // forward, 3 + q: second forward (items q).  The first powers are kept in
+  // registers; the third powers come from `t3` (pass -> value).
+  static constexpr int NTW = 3 + NL;
+  __device__ static __forceinline__ int tw_index(int k, int jl) {
+    if (k == 0) return E == 8 ? jl % R0 * (N / (8 * R0)) : jl % 8 * 6;
+    if (k == 1) return jl;
+    if (k == 2) return jl % E * (N / (8 * E));
+    const int j = jl + RL * (k - 3);
+    return E == 8 || j < 48 ? j : 0;
+  }
   struct Tw {
-    T2 inv1, inv2, fwd1, fwd2[NL];
+    T2 p[NTW];
   };
-  __device__ static __forceinline__ Tw twiddles(const T2* __restrict__ tw, int jl) {
+  // the first (pw = 1) or third (pw = 3) powers
+  __device__ static __forceinline__ Tw twiddles(const T2* __restrict__ tw, int jl, int pw) {
     Tw t;
-    t.inv1 = tw[E == 8 ? jl % R0 * (N / (8 * R0)) : jl % 8 * 6];
-    t.inv2 = tw[jl];
-    t.fwd1 = tw[jl % E * (N / (8 * E))];
 #pragma unroll
-    for (int q = 0; q < NL; ++q) t.fwd2[q] = tw[E == 8 || jl + RL * q < 48 ? jl + RL * q : 0];
+    for (int k = 0; k < NTW; ++k) t.p[k] = tw[pw * tw_index(k, jl) % N];
     return t;
   }
   // This thread's (kx, line pair) items of a field: byte offset in the field
@@ -968,7 +1004,9 @@ struct XRow {
     if (c + RL <= NP || c > N - NP) return A[li(jl) + c / 8 * 9];
     return i < NP || i > N - NP ? A[li(jl) + c / 8 * 9] : T2{0, 0};
   }
-  __device__ static __forceinline__ void inverse(T2* A, int jl, const Tw& tw, T2 (&w)[E]) {
+  template <typename T3>
+  __device__ static __forceinline__ void inverse(T2* A, int jl, const Tw& tw, const T3& t3,
+                                                 T2 (&w)[E]) {
     if constexpr (E == 8) {
       if constexpr (R0 > 1) {
 #pragma unroll
@@ -987,7 +1025,7 @@ struct XRow {
       }
 #pragma unroll
       for (int r = 0; r < 8; ++r) w[r] = R0 > 1 ? A[at(jl, r)] : packed(A, jl, RL * r);
-      if constexpr (R0 > 1) twiddle_pow<8>(w, tw.inv1, +1);
+      if constexpr (R0 > 1) twiddle_pow3<8>(w, tw.p[0], t3(0), +1);
       dft8<T, T2>(w, +1);
       wave_sync();
       const int o = li(jl / R0 * (R0 * 8) + jl % R0);
@@ -1020,7 +1058,7 @@ struct XRow {
 #pragma unroll
       for (int q = 0; q < NL; ++q)
         if (48 % RL == 0 || jl + RL * q < 48) {
-          twiddle_pow<RB>(v + q * RB, tw.inv1, +1);
+          twiddle_pow3<RB>(v + q * RB, tw.p[0], t3(0), +1);
           dft_r<RB, T, T2>(v + q * RB, +1);
           const int j = jl + RL * q, o = j / 8 * (9 * RB) + j % 8;
 #pragma unroll
@@ -1030,7 +1068,7 @@ struct XRow {
     wave_sync();
 #pragma unroll
     for (int r = 0; r < E; ++r) w[r] = A[at(jl, r)];
-    twiddle_pow<E>(w, tw.inv2, +1);
+    twiddle_pow3<E>(w, tw.p[1], t3(1), +1);
     dft_r<E, T, T2>(w, +1);
   }
   // Transform of sign s (first twiddles of sign -1) of the row whose entries
@@ -1045,8 +1083,9 @@ struct XRow {
   __device__ static __forceinline__ int last_at(int jl, int q, int r) {
     return li(jl) + RL / 8 * 9 * q + NLAST / 8 * 9 * r;
   }
-  __device__ static __forceinline__ void row_fft(T2* A, int jl, const Tw& tw, int s, T2 (&w)[E],
-                                                 T2 (&v)[NL][RLAST]) {
+  template <typename T3>
+  __device__ static __forceinline__ void row_fft(T2* A, int jl, const Tw& tw, const T3& t3, int s,
+                                                 T2 (&w)[E], T2 (&v)[NL][RLAST]) {
     dft_r<E, T, T2>(w, s);
 #pragma unroll
     for (int r = 0; r < E; ++r) A[E == 8 ? 9 * jl + r : li(6 * jl + r)] = w[r];
@@ -1058,14 +1097,14 @@ struct XRow {
       for (int r = 0; r < 8; ++r) u[r] = A[E == 8 ? at(jl, r) : li(jl + r * (N / 8))];
     }
     if constexpr (E == 8 && R0 == 1) {
-      twiddle_pow<8>(u, tw.fwd2[0], s);
+      twiddle_pow3<8>(u, tw.p[3], t3(3), s);
       dft8<T, T2>(u, s);
 #pragma unroll
       for (int r = 0; r < 8; ++r) v[0][r] = u[r];
     } else {
       wave_sync();
       if (on) {
-        twiddle_pow<8>(u, tw.fwd1, s);
+        twiddle_pow3<8>(u, tw.p[2], t3(2), s);
         dft8<T, T2>(u, s);
         const int o = jl / E * (8 * E) + jl % E;
 #pragma unroll
@@ -1077,14 +1116,16 @@ struct XRow {
         if (last_on(jl, q)) {
 #pragma unroll
           for (int r = 0; r < RLAST; ++r) v[q][r] = A[last_at(jl, q, r)];
-          twiddle_pow<RLAST>(v[q], tw.fwd2[q], s);
+          twiddle_pow3<RLAST>(v[q], tw.p[3 + q], t3(3 + q), s);
           dft_r<RLAST, T, T2>(v[q], s);
         }
     }
   }
-  __device__ static __forceinline__ void forward(T2* A, int jl, const Tw& tw, T2 (&w)[E]) {
+  template <typename T3>
+  __device__ static __forceinline__ void forward(T2* A, int jl, const Tw& tw, const T3& t3,
+                                                 T2 (&w)[E]) {
     T2 v[NL][RLAST];
-    row_fft(A, jl, tw, -1, w, v);
+    row_fft(A, jl, tw, t3, -1, w, v);
     wave_sync();
 #pragma unroll
     for (int q = 0; q < NL; ++q)
@@ -1150,12 +1191,12 @@ __global__ __launch_bounds__(256) void k_fourz_row(const double2* __restrict__ t
   const int lr = threadIdx.x / RL, jl = threadIdx.x - lr * RL;
   const long long row = (long long)blockIdx.x * ROWS + lr;
   if (row >= nrows) return;
-  const typename C::Tw twd = C::twiddles(tw, jl);
+  const typename C::Tw twd = C::twiddles(tw, jl, 1), tw3 = C::twiddles(tw, jl, 3);
   double2* p = c + row * N + jl;
   double2 w[C::E], v[C::NL][C::RLAST];
 #pragma unroll
   for (int r = 0; r < C::E; ++r) w[r] = p[RL * r];
-  C::row_fft(buf + lr * C::RS, jl, twd, iopt < 0 ? -1 : 1, w, v);
+  C::row_fft(buf + lr * C::RS, jl, twd, [&](int k) { return tw3.p[k]; }, iopt < 0 ? -1 : 1, w, v);
   const double sc = iopt < 0 ? 1.0 / N : 1.0;
 #pragma unroll
   for (int q = 0; q < C::NL; ++q)
