@@ -247,8 +247,8 @@ int zfft_blocks(const FftArgs& a);
 int xline_blocks(const FftArgs& a);
 
 int launch_zfft_inv(bool fp32, const FftArgs& a, hipStream_t st);
-// whether the run's length, tile and size take the row kernel (the caller
-// sets a.xrow)
+// whether the run's length and tile take the row kernel (the caller sets
+// a.xrow)
 bool xrow_serves(bool fp32, const FftArgs& a);
 int launch_xline(bool fp32, const FftArgs& a, hipStream_t st);
 int launch_zfft_fwd(bool fp32, const FftArgs& a, hipStream_t st);
