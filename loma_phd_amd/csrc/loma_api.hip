@@ -2014,6 +2014,7 @@ static int solve_cols(loma_run* r, const double* phi, double* v, double* dvdy,
                       const double* rK, double shift, int ncols, int mode) {
   if (!r || ncols < 0) return LOMA_ERR_ARG;
   if (ncols == 0) return LOMA_OK;
+  if (!rK) { set_error("batched solve: null rK"); return LOMA_ERR_ARG; }
   std::lock_guard<std::mutex> lk(r->ws_mu);
   int chunk = 0;
   int e = solve_ws(r, ncols, 1, &chunk);

@@ -78,3 +78,22 @@ def test_visc_pieces(gpu, my, ncols):
         assert torch.equal(b[:ncols], s[torch.arange(ncols) % PERIOD])
         assert (b[ncols:] == 7.0).all()
     run.close()
+
+
+def test_null_wavenumbers_are_refused(gpu):
+    """No wavenumbers: an error of the call, nothing launched; no columns: nothing
+    to do."""
+    import torch
+    from loma_phd_amd import capi, grid
+    run = capi.Run(48, 17, 48, grid.tanh_mesh(17, 20.0), 300.0, 0.25, 0.25)
+    x = torch.ones(3, 17, 2, dtype=torch.float64, device="cuda")
+    v = torch.full_like(x, 7.0)
+    torch.cuda.synchronize()
+    for call in (run.lapvdvhom_dev, run.solvepsi_dev):
+        with pytest.raises(capi.LomaError):
+            call(x.data_ptr(), v.data_ptr(), v.data_ptr(), None, 3)
+        call(x.data_ptr(), v.data_ptr(), v.data_ptr(), None, 0)
+    with pytest.raises(capi.LomaError):
+        run.helmholtz_dev(x.data_ptr(), v.data_ptr(), None, 1.0, 3)
+    assert (v.cpu() == 7.0).all()
+    run.close()
