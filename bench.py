@@ -33,10 +33,10 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E
 # writes 1 GiB by these sums (python3 -m loma_phd_amd.profile_step; summary
 # in profiles/rk3_step_512x513x256_hbm_traffic.md).
 MEASURED_TRAFFIC = {
-    "fp64": {"phaseA": 4.262e9, "zfft_inv": 4.775e9, "xline": 7.364e9,
-             "zfft_fwd": 6.582e9, "phaseC": 4.328e9, "phaseC2": 0.978e9},
-    "mixed": {"phaseA": 3.309e9, "zfft_inv": 2.408e9, "xline": 4.217e9,
-              "zfft_fwd": 3.327e9, "phaseC": 3.112e9, "phaseC2": 0.853e9},
+    "fp64": {"phaseA": 3.981e9, "zfft_inv": 4.179e9, "xline": 7.343e9,
+             "zfft_fwd": 5.984e9, "phaseC": 4.051e9, "phaseC2": 1.007e9},
+    "mixed": {"phaseA": 3.156e9, "zfft_inv": 2.107e9, "xline": 4.214e9,
+              "zfft_fwd": 3.024e9, "phaseC": 3.057e9, "phaseC2": 0.870e9},
 }
 
 
@@ -122,16 +122,19 @@ def measure_traffic(precision_name, timeout=240):
     return out, {k: round(v, 4) for k, v in calib.items()}
 
 
-def algorithmic_bytes(run, with_z: bool):
+def algorithmic_bytes(run, with_z: bool, step: bool = False):
     """Compulsory HBM bytes per launch of each kernel class (one substep)
     and per RK3 step: one read of every field a kernel consumes and one write
     of every field it produces (S, W, P sized; es bytes per complex transform
-    entry), nothing else.  The fields are those of foup2 (8 in, 11 out); a
-    step transforms one less each way, which the measured traffic shows."""
+    entry), nothing else.  The fields are those of foup2 (8 in, 11 out; 12 and
+    12 with Z), or with `step` those that a step transforms, one less each way
+    (dT/dx is formed from T in the x lines, and five products stand for six)."""
     S, W, P = run.S, run.W, run.P
     es = 8 if run.precision == 1 else 16
     z = 1 if with_z else 0
     nin, nout = (12, 12) if with_z else (8, 11)
+    if step:
+        nin, nout = nin - 1, nout - 1
     k = {
         # reads phi, ten13, vor, ten12, psi, T (+Z); writes phi, vor; writes
         # the transform inputs
@@ -145,8 +148,7 @@ def algorithmic_bytes(run, with_z: bool):
         # reads drho, writes psi
         "phaseC2": es * S + 16 * S,
     }
-    step = 3 * sum(k.values())
-    return k, step
+    return k, 3 * sum(k.values())
 
 
 def model_bytes_per_step(S, P, mixed: bool):
@@ -183,7 +185,7 @@ def bench_precision(cfg, st, precision, steps, warmup, prof_steps):
     run.advance(prof_steps)
     prof = run.profile_read()
     run.profile(False)
-    kb, step_bytes = algorithmic_bytes(run, cfg.scalar_z)
+    kb, step_bytes = algorithmic_bytes(run, cfg.scalar_z, step=True)
     out = dict(
         ms_per_step=total_ms / steps,
         wall_ms_per_step=wall * 1e3 / steps,
@@ -209,7 +211,7 @@ def bench_band(nsys=16384, sizes=(257, 385, 513), reps=20, seed=3):
     [1, 1e4], complex N(0,1) right-hand sides in FP32 and FP64 (FP64 factor
     and solve), through loma_band5_solve_dev.  Algorithmic bytes per system:
     n x (40 band + 16 or 8 rhs + 16 solution); the factor scratch the kernel
-    writes and reads back (2 x 40 bytes per row) is not counted."""
+    writes and reads back (2 x 32 bytes per row) is not counted."""
     import torch
     from loma_phd_amd import capi
     dev = torch.device("cuda:0")
@@ -246,8 +248,8 @@ def bench_band(nsys=16384, sizes=(257, 385, 513), reps=20, seed=3):
                 ms=round(ms, 4), algorithmic_bytes=alg,
                 achieved_GBps=round(alg / (ms * 1e-3) / 1e9, 1),
                 frac=round(alg / (ms * 1e-3) / (HBM_PEAK_GBS * 1e9), 4),
-                scratch_bytes=nsys * n * 80)
-    return dict(systems=nsys, form="per-system bands (bandec/banbks), two wavefronts per 64 systems (real and imaginary right-hand side)",
+                scratch_bytes=nsys * n * 64)
+    return dict(systems=nsys, form="per-system bands (bandec/banbks), a lane per system (complex right-hand side)",
                 results=out)
 
 
