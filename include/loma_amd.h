@@ -33,8 +33,10 @@ extern "C" {
 
 /* precision modes */
 #define LOMA_FP64 0   /* everything in double */
-#define LOMA_MIXED 1  /* FP32 transforms, nonlinear products and the
-                         y-derivatives of the vorticity/phi right-hand sides;
+#define LOMA_MIXED 1  /* FP32 transforms (dT/dx is formed from T's transformed
+                         coefficients, in FP64, and rounded once), nonlinear
+                         products and the y-derivatives of the vorticity/phi
+                         right-hand sides;
                          FP64 Helmholtz/Poisson solves, 00 modes and RK
                          accumulation */
 
@@ -181,7 +183,13 @@ int loma_profile_read(loma_run *run, double *total_ms, int *counts, int nclasses
 
 /* ---- per-operator entry points (device pointers, double) --------------- */
 /* All act on ncols complex y-columns of length my stored back to back
- * (interleaved re/im doubles), in place allowed, on the run's stream. */
+ * (interleaved re/im doubles), in place allowed, on the run's stream.  The
+ * solves (loma_lapvdvhom_dev, loma_solvepsi_dev, loma_helmholtz_dev,
+ * loma_visc_dev) factor one matrix (visc: two) per column into a device
+ * workspace, 2,560 bytes each per row of a lane (ceil(my/64) rows, at least
+ * 3), at most 256 MiB; larger batches go through it in pieces.  The workspace
+ * is allocated by a run's first such call, grown by larger ones and freed with
+ * the run; it is outside loma_footprint and loma_dims. */
 int loma_deryr2_dev(loma_run *run, const double *u, double *du, int ncols);  /* cfdiff.f:518 */
 int loma_deryyr2_dev(loma_run *run, const double *u, double *du, int ncols); /* cfdiff.f:735 */
 /* rK per column (double[ncols]) */
@@ -281,8 +289,9 @@ int loma_band5_solve_dev(const double *band, void *rhs, double *x, int n,
  * under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  Same arguments, kernel and results; the scratch is a fixed
  * array in the library's code object, 4,194,304 doubles (32 MiB) that every
- * GPU the library runs on holds until the process ends, so n*5*nsys must not
- * exceed 4,194,304 (LOMA_ERR_ARG otherwise; e.g. 1635 systems at n = 513).
+ * GPU the library runs on holds until the process ends; n*5*nsys must not
+ * exceed 4,194,304 (LOMA_ERR_ARG otherwise; e.g. 1635 systems at n = 513), the
+ * limit this entry has always had, one double a row more than it uses.
  * Calls that overlap on one GPU share that array and race. */
 int loma_band5_solve_dev_noalloc(const double *band, void *rhs, double *x, int n,
                                  int nsys, int rhs_fp32, void *stream);

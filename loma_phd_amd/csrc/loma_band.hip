@@ -219,7 +219,8 @@ int launch_band5(const double* band, const void* rhs, double* x, double* scratch
 // GPU the library runs on holds until the process ends.  Host code never
 // passes the array's name to a kernel (on the host it is only a stand-in
 // symbol); it uses the device address that hipGetSymbolAddress returns for
-// the current device, kept per device in g_scr_dev.
+// the current device, kept per device in g_scr_dev.  A row takes four doubles;
+// the limit of five, n*5*nsys, is the entry's own and stays.
 constexpr size_t BAND5_SCRATCH_DOUBLES = (size_t)1 << 22;  // 4194304 doubles, 32 MiB
 static __device__ __align__(256) double scratch[BAND5_SCRATCH_DOUBLES];
 

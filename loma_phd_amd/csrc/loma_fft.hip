@@ -594,8 +594,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LOMA_ZF_WPE
 }
 
 // ------------------------------------------------------------------------
-// x lines: inverse x transform of the 8 (12 with Z) transform inputs, phys2
-// algebra, forward x transform of the 11 (12) outputs, for 2*pairs lines
+// x lines at the lengths of the run-time plan: inverse x transform of the 7 (11
+// with Z) transform inputs, phys2 algebra, forward x transform of the 10 (11)
+// outputs (foup2: 8 and 11), for 2*pairs lines
 // (fixed z, consecutive y) per 256-thread workgroup.  Two real lines share
 // one complex FFT.  The algebra runs in two passes so that only rho*u_i, T
 // and one accumulator per point stay in registers:
@@ -650,10 +651,11 @@ __device__ __forceinline__ void xl_fetch(const FftArgs& a, const T2* __restrict_
 
 // Fields per x transform.  The rows of field f are f*pairs ..
 // f*pairs+pairs-1, so one transform of 2*pairs rows keeps every thread of
-// a radix pass busy where pairs alone is too few rows: FP64 at 512 points
-// has 2 pairs, 128 radix-8 butterflies for 256 threads (two fields per
-// transform measured 5.13 against 5.58 ms per x-line launch at
-// 512x513x256).  FP32 has 4 pairs and gains nothing from two fields.
+// a radix pass busy where pairs alone is too few rows: FP64 at 480 points
+// has 2 pairs, 120 radix-8 butterflies for 256 threads (two fields per
+// transform 2.65 against 3.39 ms an x-line launch at 480x257x240, 0.143
+// against 0.176 at 100x129x90).  FP32, with 4 pairs, carries one (2.11 ms;
+// two would take 1.90, and 0.092 instead of 0.109 at 100x129x90).
 #ifndef LOMA_XL_DUAL64
 #define LOMA_XL_DUAL64 1
 #endif
@@ -665,9 +667,10 @@ constexpr int xl_nf() {
   return (sizeof(T) == 8 ? LOMA_XL_DUAL64 : LOMA_XL_DUAL32) ? 2 : 1;
 }
 // x-line LDS rows: one pad entry after every eight (lds_i<1>) spreads the
-// strided butterfly writes of the first two radix-8 passes over the banks.
-// FP64 (16-byte entries): 4.91 against 5.20 ms per launch at 512x513x256;
-// FP32 measured slower padded (3.03 against 2.90 ms) and stays unpadded.
+// strided butterfly writes of the first radix-8 passes over the banks.  FP64
+// (16-byte entries): 2.65 against 2.69 ms a launch at 480x257x240, but 0.143
+// against 0.132 at 100x129x90; FP32 is slower padded (2.19 against 2.11 and
+// 0.121 against 0.109 ms) and stays unpadded.
 #ifndef LOMA_XL_PAD64
 #define LOMA_XL_PAD64 1
 #endif
@@ -830,8 +833,9 @@ __device__ __forceinline__ XlRk xl_rk(double dt, int rkstep) {
 }
 
 // Compiled for two waves per SIMD (LOMA_XL_WPE; FP64 always): at three,
-// FP64 spills heavily (and its Z-transport build gave wrong results), and
-// FP32 spills enough to measure slower (3.33 vs 3.22 ms at 512x513x256).
+// FP64 spilled heavily (and its Z-transport build gave wrong results), and
+// FP32 spilled enough to measure slower (3.33 vs 3.22 ms at 512x513x256, when
+// this kernel served 512 points).
 template <typename T, bool WZ, int EPT>
 __global__ __launch_bounds__(XL_THREADS)
 __attribute__((amdgpu_waves_per_eu(XL_THREADS == 512 ? 4 : (sizeof(T) == 8 ? 2 : LOMA_XL_WPE)))) void k_xline(FftArgs a) {
@@ -1182,8 +1186,8 @@ __attribute__((amdgpu_waves_per_eu(2))) void k_xrow_batch(
 // fourz on standalone rows (FFTPACK convention), for the per-operator API.
 // Lengths of XRow: RL lanes of a wavefront per row, from and to HBM in
 // registers (runs of RL entries), two exchanges through the row's LDS and no
-// workgroup barrier: 87,210 rows of 256 take 143 us, the rate of a copy, where
-// one workgroup a row took 321
+// workgroup barrier: 87,210 rows of 256 take 144 us, 5.0 TB/s where a large copy
+// reaches 5.6; one workgroup a row took 321
 template <int N>
 __global__ __launch_bounds__(256) void k_fourz_row(const double2* __restrict__ tw, double2* c,
                                                    int nrows, int iopt) {

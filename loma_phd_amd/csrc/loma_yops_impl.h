@@ -209,8 +209,7 @@ __global__ __launch_bounds__(256) void k_lapvdvhom(YTab T, const double* lu, int
 // visc (trunk/mixing/src/laps.f:535-857) for a batch of mode columns, with
 // the mixing-layer boundary functions (laps.f:893-1060).  lu1 / lu2: per
 // column LU of the Dirichlet Helmholtz matrices dt22 - rk1 dt21 and
-// dt22 - rk2 dt21; bc2: per column {w0.h1, w0.h2, w1.h1, w1.h2} of the rk2
-// homogeneous solutions (w0, w1 the d/dy functionals at the ends).
+// dt22 - rk2 dt21.
 //   omega = (D2 - rk1)^{-1} vorwk with omega = 0 at both ends (C_ome = 1,
 //     C_dyo = 0 make the 2x2 boundary system the identity);
 //   phi   = (D2 - rk1)^{-1} phiwk, zero at both ends (C_phi rows bot2/top2);
